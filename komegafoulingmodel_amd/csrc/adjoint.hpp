@@ -18,7 +18,7 @@
 // between two columns plus a weighted wall-shear integral is handled by
 // kernels over a compact list of objective nodes.
 #pragma once
-#include "kernels.hpp"
+#include "solver.hpp"
 
 namespace kofm {
 namespace dev {
@@ -561,28 +561,30 @@ __global__ __launch_bounds__(kBlockX) void koTranspose(const uint16_t* __restric
   }
 }
 
-// r = b - A x, rh = r for both systems; partials (r, r).
-__global__ __launch_bounds__(kBlockX) void bicgResidual(const uint16_t* __restrict__ mask, BicgVecs V,
-                                                        KOParams p) {
-  double a[2][2] = {{0., 0.}, {0., 0.}};
-  forOwnTiles(p, [&](int x, int y) {
+// r = b - A x of both systems; sums (r, r).
+__global__ __launch_bounds__(kStripX) void solveResidual(SolvePair P, const double* __restrict__ bk,
+                                                         const double* __restrict__ bo, KOParams p) {
+  Chunk c;
+  if (!chunkOf(P.sys[0].s, p.nX, p.nY, c)) return;
+  Sum acc[2]{};
+  forChunk(c, [&](int x, int y) {
     const size_t g = size_t(x) + size_t(p.XF) * y;
-    if (mask[g] & kSolid) return;
+    if (P.sys[0].mask[g] & kSolid) return;
     size_t nb[4];
     nbIndex(p, x, g, nb);
 #pragma unroll
     for (int v = 0; v < 2; v++) {
-      const double* A = V.A[v];
-      const double* X = V.x[v];
+      const double* A = P.sys[v].A;
+      const double* X = P.sys[v].x;
       const double ax = X[g] + (A[g] * X[nb[0]] + A[g + p.D] * X[nb[1]] + A[g + 2 * p.D] * X[nb[2]] +
                                 A[g + 3 * p.D] * X[nb[3]]);
-      const double r = V.b[v][g] - ax;
-      V.r[v][g] = r;
-      V.rh[v][g] = r;
-      a[v][0] += r * r;
+      const double r = (v == 0 ? bk : bo)[g] - ax;
+      P.sys[v].r[0][g] = r;
+      acc[v].add(r * r);
     }
   });
-  blockPartials(a, V.partial);
+  writePartial<kStripX>(P.sys[0], c.T, 0, acc[0], Sum{});
+  writePartial<kStripX>(P.sys[1], c.T, 0, acc[1], Sum{});
 }
 
 // Step 2: adjoint of the row assembly.

@@ -23,6 +23,7 @@
 #include "kernels.hpp"
 #include "nusselt.hpp"
 #include "removal.hpp"
+#include "solver.hpp"
 #include "walls.hpp"
 
 namespace kofm {
@@ -123,7 +124,7 @@ class EngineT final : public Engine {
     HIP_TRY(ux_.alloc(D * sizeof(R)));
     HIP_TRY(uy_.alloc(D * sizeof(R)));
     if (ko_) {
-      for (Buffer* b : {&K_, &O_, &nut_, &wallD_, &Dk_, &Do_, &F1_, &bk_, &bo_})
+      for (Buffer* b : {&K_, &O_, &nut_, &wallD_, &Dk_, &Do_, &F1_})
         HIP_TRY(b->alloc(D * sizeof(double)));
       HIP_TRY(S_.alloc(3 * D * sizeof(double)));
       HIP_TRY(dkdo_.alloc(2 * D * sizeof(double)));
@@ -133,17 +134,16 @@ class EngineT final : public Engine {
       HIP_TRY(Kprev_.alloc(D * sizeof(double)));
       HIP_TRY(Oprev_.alloc(D * sizeof(double)));
     }
-    HIP_TRY(status_.alloc(sizeof(dev::BicgState)));
+    HIP_TRY(status_.alloc(2 * sizeof(dev::SolveState)));
     // pinned, so that the per-step poll of the solver state is one DMA
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&hostStatus_), sizeof(dev::BicgState),
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&hostStatus_), 2 * sizeof(dev::SolveState),
                           hipHostMallocDefault));
     if (ko_)
-      for (int v = 0; v < 2; v++)
-        for (Buffer* b : {&kr_[v], &krh_[v], &kp_[v][0], &kp_[v][1], &kv_[v][0], &kv_[v][1], &ks_[v], &kt_[v]})
-          HIP_TRY(b->alloc(D * sizeof(double)));
-    const size_t nTiles = size_t((nX_ + dev::kBlockX - 1) / dev::kBlockX) * nY_;
-    const size_t nblk = 8 * ((nTiles + 7) / 8);
-    HIP_TRY(partial_.alloc(4 * nblk * sizeof(double)));
+      for (Buffer* b : solverBuffers()) HIP_TRY(b->alloc(D * sizeof(double)));
+    strips_ = dev::stripsFor(nX_, nY_);
+    // [system][pass parity][block][2] sums, and the pass states behind them
+    HIP_TRY(partial_.alloc(8 * size_t(strips_.nblk) * sizeof(double2)));
+    HIP_TRY(passState_.alloc(4 * sizeof(dev::SolveState)));
     HIP_TRY(redPartial_.alloc(dev::kReducePartials * sizeof(double)));
     HIP_TRY(redOut_.alloc(sizeof(double)));
     return 0;
@@ -331,10 +331,8 @@ class EngineT final : public Engine {
     // keep their coupling to a solid neighbour (whose value is zero): a node
     // that has turned solid must not keep the Krylov vectors' old values
     if (ko_)
-      for (int v = 0; v < 2; v++)
-        for (Buffer* b : {&kr_[v], &krh_[v], &kp_[v][0], &kp_[v][1], &kv_[v][0], &kv_[v][1],
-                          &ks_[v], &kt_[v]})
-          HIP_TRY(hipMemsetAsync(b->as<void>(), 0, b->bytes(), stream_));
+      for (Buffer* b : solverBuffers())
+        HIP_TRY(hipMemsetAsync(b->as<void>(), 0, b->bytes(), stream_));
     if (ko_)  // dXArr from the clean walls' spacings (clVariablesLS::update)
       HIP_TRY(hipMemcpyAsync(dX_.as<void>(), dX0_.as<void>(), 4 * D * sizeof(double),
                              hipMemcpyDeviceToDevice, stream_));
@@ -728,13 +726,13 @@ class EngineT final : public Engine {
   }
 
   int solverStats(SolverStats& s, std::string& err) override {
-    dev::BicgState st;
-    HIP_TRY(hipMemcpyAsync(&st, status_.as<void>(), sizeof(st), hipMemcpyDeviceToHost, stream_));
+    dev::SolveState st[2];
+    HIP_TRY(hipMemcpyAsync(st, status_.as<void>(), sizeof(st), hipMemcpyDeviceToHost, stream_));
     HIP_TRY(hipStreamSynchronize(stream_));
     for (int v = 0; v < 2; v++) {
-      s.iters[v] = st.iters[v];
-      s.res0[v] = st.r0[v];
-      s.res[v] = st.rn[v];
+      s.iters[v] = st[v].iters;
+      s.res0[v] = st[v].r0;
+      s.res[v] = st[v].rn;
     }
     s.nan = nanCount_;
     s.stepsPerLB = stepsPerLB_;
@@ -742,11 +740,11 @@ class EngineT final : public Engine {
     s.batches = batchCount_;
     s.rollbacks = rollbackCount_;
     if (tOn_) {
-      HIP_TRY(hipMemcpyAsync(&st, statusT_.as<void>(), sizeof(st), hipMemcpyDeviceToHost, stream_));
+      HIP_TRY(hipMemcpyAsync(st, statusT_.as<void>(), sizeof(st[0]), hipMemcpyDeviceToHost, stream_));
       HIP_TRY(hipStreamSynchronize(stream_));
-      s.tIters = st.iters[0];
-      s.tRes0 = st.r0[0];
-      s.tRes = st.rn[0];
+      s.tIters = st[0].iters;
+      s.tRes0 = st[0].r0;
+      s.tRes = st[0].rn;
       s.tStepsPerLB = tSteps_;
       s.tTimeStep = tDt_;
       s.nan += tNan_;
@@ -773,13 +771,13 @@ class EngineT final : public Engine {
     if (!(q.prTurb > 0.) || !(q.dt > 0.) || q.maxIters < 1)
       return fail(err, "thermal parameters: need Pr_t > 0, dt > 0 and max iterations >= 1");
     const size_t D = size_t(D_);
-    for (Buffer* b : {&T_, &Tprev_, &bt_, &tr_, &trh_, &tp_[0], &tp_[1], &tv_[0], &tv_[1], &ts_, &tt_})
+    for (Buffer* b : {&T_, &Tprev_, &tr_[0], &tr_[1], &tr_[2], &tp_[0], &tp_[1], &tv_[0], &tv_[1], &tt_})
       HIP_TRY(b->alloc(D * sizeof(double)));
     HIP_TRY(At_.alloc(4 * D * sizeof(double)));
     HIP_TRY(tmask_.alloc(D * sizeof(uint16_t)));
-    HIP_TRY(statusT_.alloc(sizeof(dev::BicgState)));
+    HIP_TRY(statusT_.alloc(sizeof(dev::SolveState)));
     if (!hostStatusT_)
-      HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&hostStatusT_), sizeof(dev::BicgState),
+      HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&hostStatusT_), sizeof(dev::SolveState),
                             hipHostMallocDefault));
     std::vector<uint16_t> m(D, 0);
     std::vector<double> T(D, 0.);
@@ -828,10 +826,7 @@ class EngineT final : public Engine {
     if (!tOn_) return fail(err, "initialise the temperature solve first");
     if (!haveState_) return fail(err, "state not initialised");
     auto kp = koParams();
-    const dim3 blk(dev::kBlockX);
-    const int nsb = solverBlocks();
-    auto* st = statusT_.as<dev::BicgState>();
-    const dev::BicgVecs V = thermalVecs();
+    const dev::SolvePair P = thermalSystem();
     for (int c = 0; c < n; c++) {
       if (++tQuiet_ >= kDtQuiet) {
         tQuiet_ = 0;
@@ -843,19 +838,15 @@ class EngineT final : public Engine {
       bool first = true;
       int sub = 0;
       while (sub < tSteps_) {
-        hipLaunchKernelGGL(dev::bicgResetT, dim3(1), dim3(64), 0, stream_, st, tRel_, tAbs_, tMaxIt_);
-        hipLaunchKernelGGL((dev::thermalCoeffs<R>), dim3(nsb), blk, 0, stream_,
-                           (const uint16_t*)tmask_.as<uint16_t>(),
+        hipLaunchKernelGGL((dev::thermalCoeffs<R>), solveGrid(1), dim3(dev::kStripX), 0, stream_,
                            (const uint16_t*)mask_.as<uint16_t>(), (const double*)dX0_.as<double>(),
                            (const double*)nut_.as<double>(), (const R*)ux_.as<R>(),
-                           (const R*)uy_.as<R>(), first ? Tprev_.as<double>() : nullptr, V, tpar_,
+                           (const R*)uy_.as<R>(), first ? Tprev_.as<double>() : nullptr, P, tpar_,
                            tDt_, kp);
-        hipLaunchKernelGGL(dev::bicgScalars, dim3(1), dim3(1024), 0, stream_,
-                           (const double*)partial_.as<double>(), nsb, st, 0);
         const int batch = std::min(std::max(1, tIters_), 8);
-        enqueueIters(batch, V, tmask_.as<uint16_t>(), st);
+        enqueueIters(P, 1, 0, batch);
         bool nan = false;
-        int rc = thermalFinish(batch, V, nan, err);
+        int rc = thermalFinish(batch, P, nan, err);
         if (rc) return rc;
         first = false;
         if (tInjectNan_) {
@@ -1206,14 +1197,15 @@ class EngineT final : public Engine {
   bool ko_;
   hipStream_t stream_ = nullptr;
   Buffer fA_, fB_, mask_, ibbIdx_, ibbQ_, rho_, ux_, uy_;
-  Buffer K_, O_, nut_, S_, wallD_, Dk_, Do_, F1_, dkdo_, dX_, Ak_, Ao_, bk_, bo_;
+  Buffer K_, O_, nut_, S_, wallD_, Dk_, Do_, F1_, dkdo_, dX_, Ak_, Ao_;
   Buffer ntype_, dX0_;  // node types and clean-wall spacings (moving-wall update)
   std::vector<double> wallC0_;  // the wall points of the built (clean) geometry
   bool wallsMoved_ = false;     // the walls were updated since the geometry was built
   Buffer Kprev_, Oprev_;  // k, omega at the start of the step (restart point)
-  Buffer kr_[2], krh_[2], kp_[2][2], kv_[2][2], ks_[2], kt_[2];  // FP64 BiCGStab vectors, [0] = k
+  Buffer kr_[2][3], kp_[2][2], kv_[2][2], kt_[2];  // FP64 BiCGStab vectors, [0] = k
   Buffer ss_, cfss_, tau_, sInd_, wts_, tauBL_;
-  Buffer status_, partial_, redPartial_, redOut_;
+  Buffer status_, passState_, partial_, redPartial_, redOut_;
+  dev::Strips strips_{};  // the solver passes' blocks
   int lastIters_ = 1;  // iterations the previous k-omega solve needed
   // k-omega time step control (kOmega.cpp:31-73, 387-414): sub-steps per LB
   // step, their time step, steps since the last change, and non-finite
@@ -1236,8 +1228,8 @@ class EngineT final : public Engine {
   // mask of the clean geometry (solid = not a row), the solver's own vectors
   // (the fouling layer is a row here but solid for k-omega, whose vectors
   // must read zero there) and state, the time step control
-  Buffer T_, Tprev_, At_, bt_, tmask_, statusT_, tr_, trh_, tp_[2], tv_[2], ts_, tt_;
-  dev::BicgState* hostStatusT_ = nullptr;
+  Buffer T_, Tprev_, At_, tmask_, statusT_, tr_[3], tp_[2], tv_[2], tt_;
+  dev::SolveState* hostStatusT_ = nullptr;
   dev::TParams tpar_{};
   double tRel_ = 1e-4, tAbs_ = 1e-7, tDt_ = 1.;
   int tMaxIt_ = 1000, tSteps_ = 1, tQuiet_ = 0, tIters_ = 1, tNan_ = 0;
@@ -1256,7 +1248,7 @@ class EngineT final : public Engine {
   bool remValid_ = false;
   static constexpr int kDtQuiet = 20;              // kOmega.h:22 timeBtwIncreaseTimeStep
   static constexpr int kMaxStepsPerLB = 1 << 16;   // halvings give up beyond this
-  dev::BicgState* hostStatus_ = nullptr;  // pinned copy of the solver state
+  dev::SolveState* hostStatus_ = nullptr;  // pinned copy of both systems' states
   // adjoint: checkpoints of the objective run, the recomputed segment, the
   // two adjoint population levels, per-link buffers and the objective nodes
   struct ObjectiveRun {
@@ -1388,14 +1380,14 @@ class EngineT final : public Engine {
   }
 
   // The transposed systems share the forward solver's work vectors.
-  dev::BicgVecs adjVecs() const {
-    dev::BicgVecs V = bicgVecs();
+  dev::SolvePair adjSystems() const {
+    dev::SolvePair P = koSystems();
     for (int v = 0; v < 2; v++) {
-      V.x[v] = adjPlane(kALam + v);
-      V.A[v] = adjPlane(v == 0 ? kATk : kATo);
-      V.b[v] = adjPlane(v == 0 ? kAKb : kAOb);
+      P.sys[v].x = adjPlane(kALam + v);
+      P.sys[v].A = adjPlane(v == 0 ? kATk : kATo);
+      P.sys[v].atol = 0.;
     }
-    return V;
+    return P;
   }
 
   struct Copy {
@@ -1541,7 +1533,7 @@ class EngineT final : public Engine {
       launchLBBlock<true>(lbBlock_, lbNpt_, p, seg_[m]->template as<S>(), seg_[m + 1]->template as<S>());
       const int batch = std::min(std::max(1, lastIters_), 8);
       enqueueKoHead();
-      enqueueIters(batch);
+      enqueueIters(koSystems(), 2, 0, batch);
       bool nan = false;
       int rc = koFinish(batch, nan, err);
       if (rc) return rc;
@@ -1553,11 +1545,9 @@ class EngineT final : public Engine {
     }
     auto kp = koParams();
     const dim3 grid(8 * kp.tiles.per), blk(dev::kBlockX);
-    const int nsb = solverBlocks();
     const dim3 og((on.n + 63) / 64), ig((nIbbNodes_ + 63) / 64);
     const dev::KOAdjoint ka = koAdj();
-    const dev::BicgVecs V = adjVecs();
-    auto* st = status_.as<dev::BicgState>();
+    const dev::SolvePair P = adjSystems();
     const uint16_t* mask = mask_.as<uint16_t>();
     const int frozen = (run_.obj.flags & KOFM_ADJOINT_FROZEN_TURBULENCE) ? 1 : 0;
     for (int m = len - 1; m >= 0; m--) {
@@ -1566,14 +1556,11 @@ class EngineT final : public Engine {
         // 1. the transposed implicit systems, warm-started from the last solution
         hipLaunchKernelGGL(dev::koTranspose, grid, blk, 0, stream_, mask, (const double*)tapePlane(m, kTAk),
                            (const double*)tapePlane(m, kTAo), adjPlane(kATk), adjPlane(kATo), kp);
-        hipLaunchKernelGGL(dev::bicgReset, dim3(1), dim3(64), 0, stream_, st, par_.relTol[0], 0.,
-                           par_.maxIters[0], par_.relTol[1], 0., par_.maxIters[1]);
-        hipLaunchKernelGGL(dev::bicgResidual, dim3(nsb), blk, 0, stream_, mask, V, kp);
-        hipLaunchKernelGGL(dev::bicgScalars, dim3(1), dim3(1024), 0, stream_,
-                           (const double*)partial_.as<double>(), nsb, st, 0);
+        hipLaunchKernelGGL(dev::solveResidual, solveGrid(1), dim3(dev::kStripX), 0, stream_, P,
+                           (const double*)adjPlane(kAKb), (const double*)adjPlane(kAOb), kp);
         const int batch = std::min(std::max(1, adjIters_), 8);
-        enqueueIters(batch, V);
-        int rc = solveFinish(batch, V, adjIters_, err);
+        enqueueIters(P, 2, 0, batch);
+        int rc = solveFinish(batch, P, adjIters_, err);
         if (rc) return rc;
         // 2, 3: rows and diffusivities
         hipLaunchKernelGGL((dev::koRowsAdjoint<R>), grid, blk, 0, stream_, mask, wallD_.as<double>(),
@@ -2262,48 +2249,70 @@ class EngineT final : public Engine {
   }
 
  private:
-  // The solver's device vectors.
-  dev::BicgVecs bicgVecs() const {
-    using K = double;
-    dev::BicgVecs V;
-    V.x[0] = K_.as<K>();
-    V.x[1] = O_.as<K>();
-    V.A[0] = Ak_.as<K>();
-    V.A[1] = Ao_.as<K>();
-    V.b[0] = bk_.as<K>();
-    V.b[1] = bo_.as<K>();
-    for (int v = 0; v < 2; v++) {
-      V.r[v] = kr_[v].as<K>();
-      V.rh[v] = krh_[v].as<K>();
-      V.s[v] = ks_[v].as<K>();
-      V.t[v] = kt_[v].as<K>();
-      for (int c = 0; c < 2; c++) {
-        V.p[v][c] = kp_[v][c].as<K>();
-        V.v[v][c] = kv_[v][c].as<K>();
-      }
-    }
-    V.partial = partial_.as<double>();
-    V.prev[0] = V.prev[1] = nullptr;
-    return V;
+  // Every vector of the k and omega solves.
+  std::vector<Buffer*> solverBuffers() {
+    std::vector<Buffer*> all;
+    for (int v = 0; v < 2; v++)
+      for (Buffer* b : {&kr_[v][0], &kr_[v][1], &kr_[v][2], &kp_[v][0], &kp_[v][1], &kv_[v][0],
+                        &kv_[v][1], &kt_[v]})
+        all.push_back(b);
+    return all;
   }
 
-  // The temperature system as system 0 of the solver (system 1 is never
-  // touched: its zero partials end it at stage 0).
-  dev::BicgVecs thermalVecs() const {
-    dev::BicgVecs V = bicgVecs();
-    V.x[0] = V.x[1] = T_.as<double>();
-    V.A[0] = V.A[1] = At_.as<double>();
-    V.b[0] = V.b[1] = bt_.as<double>();
-    V.r[0] = V.r[1] = tr_.as<double>();
-    V.rh[0] = V.rh[1] = trh_.as<double>();
-    V.s[0] = V.s[1] = ts_.as<double>();
-    V.t[0] = V.t[1] = tt_.as<double>();
-    for (int c = 0; c < 2; c++) {
-      V.p[0][c] = V.p[1][c] = tp_[c].as<double>();
-      V.v[0][c] = V.v[1][c] = tv_[c].as<double>();
+  // What the systems of this lattice have in common.
+  dev::SolveSys systemBase(int v) const {
+    dev::SolveSys y{};
+    y.mask = mask_.as<uint16_t>();
+    y.st = passState_.as<dev::SolveState>() + 2 * v;
+    y.partial = partial_.as<double2>() + size_t(v) * 4 * strips_.nblk;
+    y.nX = nX_;
+    y.nY = nY_;
+    y.XF = XF_;
+    y.D = D_;
+    y.s = strips_;
+    return y;
+  }
+
+  // The k and omega systems.
+  dev::SolvePair koSystems() const {
+    dev::SolvePair P;
+    for (int v = 0; v < 2; v++) {
+      dev::SolveSys y = systemBase(v);
+      y.x = (v == 0 ? K_ : O_).as<double>();
+      y.A = (v == 0 ? Ak_ : Ao_).as<double>();
+      for (int c = 0; c < 3; c++) y.r[c] = kr_[v][c].as<double>();
+      for (int c = 0; c < 2; c++) {
+        y.p[c] = kp_[v][c].as<double>();
+        y.v[c] = kv_[v][c].as<double>();
+      }
+      y.t = kt_[v].as<double>();
+      y.out = status_.as<dev::SolveState>() + v;
+      y.rtol = par_.relTol[v];
+      y.atol = par_.absTol[v];
+      y.maxit = par_.maxIters[v];
+      P.sys[v] = y;
     }
-    V.prev[0] = V.prev[1] = nullptr;
-    return V;
+    return P;
+  }
+
+  // The temperature system.
+  dev::SolvePair thermalSystem() const {
+    dev::SolveSys y = systemBase(0);
+    y.mask = tmask_.as<uint16_t>();
+    y.x = T_.as<double>();
+    y.A = At_.as<double>();
+    for (int c = 0; c < 3; c++) y.r[c] = tr_[c].as<double>();
+    for (int c = 0; c < 2; c++) {
+      y.p[c] = tp_[c].as<double>();
+      y.v[c] = tv_[c].as<double>();
+    }
+    y.t = tt_.as<double>();
+    y.out = statusT_.as<dev::SolveState>();
+    y.rtol = tRel_;
+    y.atol = tAbs_;
+    y.maxit = tMaxIt_;
+    y.crit = 1;
+    return {{y, y}};
   }
 
   // The links whose search box reaches each (column, wall) slot, in the
@@ -2421,26 +2430,25 @@ class EngineT final : public Engine {
 
   // Polls the temperature solve until it is done (adding chunks of four
   // iterations); nan reports a non-finite or jumping residual.
-  int thermalFinish(int launched, const dev::BicgVecs& V, bool& nan, std::string& err) {
+  int thermalFinish(int launched, const dev::SolvePair& P, bool& nan, std::string& err) {
     int it = launched;
-    auto* st = statusT_.as<dev::BicgState>();
-    const dev::BicgState& hs = *hostStatusT_;
+    const dev::SolveState& hs = *hostStatusT_;
     while (true) {
-      HIP_TRY(hipMemcpyAsync(hostStatusT_, st, sizeof(hs), hipMemcpyDeviceToHost, stream_));
+      HIP_TRY(hipMemcpyAsync(hostStatusT_, statusT_.as<void>(), sizeof(hs), hipMemcpyDeviceToHost, stream_));
       HIP_TRY(hipStreamSynchronize(stream_));
-      if (hs.nan || (hs.done[0] && hs.done[1]) || it >= tMaxIt_) break;
+      if (hs.nan || hs.done || it >= tMaxIt_) break;
       const int k = std::min(4, tMaxIt_ - it);
-      enqueueIters(k, V, tmask_.as<uint16_t>(), st);
+      enqueueIters(P, 1, it, k);
       it += k;
     }
     nan = hs.nan != 0;
-    tIters_ = hs.iters[0];
+    tIters_ = hs.iters;
     HIP_TRY(hipGetLastError());
     return 0;
   }
 
-  // the solver kernels walk their XCD's tiles with a fixed block count
-  int solverBlocks() const { return std::min(8 * koParams().tiles.per, 2048); }
+  // the solver passes of n systems
+  dim3 solveGrid(int n) const { return dim3(unsigned(8 * strips_.per), unsigned(n)); }
 
   // kOmega::Solve (kOmega.cpp:31-73), first part: diffusivities, then the
   // coefficients with the first residual and the solver's stage 0.  The
@@ -2449,47 +2457,35 @@ class EngineT final : public Engine {
   void enqueueKoHead(bool savePrev = false) {
     auto kp = koParams();
     const dim3 grid(8 * kp.tiles.per), blk(dev::kBlockX);
-    const int nsb = solverBlocks();
     using K = double;
     hipLaunchKernelGGL((dev::koDiffusivities<R>), grid, blk, 0, stream_, mask_.as<uint16_t>(),
                        K_.as<K>(), O_.as<K>(), nut_.as<K>(), wallD_.as<K>(), Dk_.as<K>(),
                        Do_.as<K>(), F1_.as<K>(), dkdo_.as<K>(), rho_.as<R>(), dX_.as<K>(), kp);
-    auto* st = status_.as<dev::BicgState>();
-    hipLaunchKernelGGL(dev::bicgReset, dim3(1), dim3(64), 0, stream_, st, par_.relTol[0],
-                       par_.absTol[0], par_.maxIters[0], par_.relTol[1], par_.absTol[1],
-                       par_.maxIters[1]);
-    dev::BicgVecs V = bicgVecs();
-    if (savePrev) {
-      V.prev[0] = Kprev_.as<K>();
-      V.prev[1] = Oprev_.as<K>();
-    }
-    hipLaunchKernelGGL((dev::koCoeffs<R>), dim3(nsb), blk, 0, stream_, mask_.as<uint16_t>(),
+    hipLaunchKernelGGL((dev::koCoeffs<R>), solveGrid(1), dim3(dev::kStripX), 0, stream_,
                        nut_.as<K>(), Dk_.as<K>(), Do_.as<K>(), F1_.as<K>(), dkdo_.as<K>(),
                        S_.as<K>(), rho_.as<R>(), ux_.as<R>(), uy_.as<R>(), dX_.as<K>(),
-                       wallD_.as<K>(), V, kp);
-    hipLaunchKernelGGL(dev::bicgScalars, dim3(1), dim3(1024), 0, stream_,
-                       (const double*)partial_.as<double>(), nsb, st, 0);
+                       wallD_.as<K>(), savePrev ? Kprev_.as<K>() : nullptr,
+                       savePrev ? Oprev_.as<K>() : nullptr, koSystems(), kp);
   }
 
-  // k BiCGStab iterations of both systems (launches past convergence return
-  // at once).
-  void enqueueIters(int k) { enqueueIters(k, bicgVecs()); }
-  void enqueueIters(int k, const dev::BicgVecs& V) {
-    enqueueIters(k, V, mask_.as<uint16_t>(), status_.as<dev::BicgState>());
-  }
-  void enqueueIters(int k, const dev::BicgVecs& V, const uint16_t* mask, dev::BicgState* st) {
-    auto kp = koParams();
-    const dim3 sgrid(solverBlocks()), blk(dev::kBlockX);
-    const int nsb = solverBlocks();
-    const double* part = partial_.as<double>();
-    for (int c = 0; c < k; c++) {
-      hipLaunchKernelGGL(dev::bicgPV, sgrid, blk, 0, stream_, mask, V, (const dev::BicgState*)st, kp);
-      hipLaunchKernelGGL(dev::bicgScalars, dim3(1), dim3(1024), 0, stream_, part, nsb, st, 1);
-      hipLaunchKernelGGL(dev::bicgST, sgrid, blk, 0, stream_, mask, V, (const dev::BicgState*)st, kp);
-      hipLaunchKernelGGL(dev::bicgScalars, dim3(1), dim3(1024), 0, stream_, part, nsb, st, 2);
-      hipLaunchKernelGGL(dev::bicgXR, sgrid, blk, 0, stream_, mask, V, (const dev::BicgState*)st, kp);
-      hipLaunchKernelGGL(dev::bicgScalars, dim3(1), dim3(1024), 0, stream_, part, nsb, st, 3);
+  // BiCGStab iterations it0 .. it0 + k - 1 of n systems (passes of a system
+  // that is done return at once), then their states; with flags, solveFinish's
+  // summary.
+  void enqueueIters(const dev::SolvePair& P, int n, int it0, int k, int* flags = nullptr) {
+    const dim3 grid = solveGrid(n), blkA(dev::kStripThreads), blkU(dev::kStripX);
+    for (int it = it0; it < it0 + k; it++) {
+      const int par = (3 * it) & 1;  // the parity alternates from pass to pass
+      if (it == 0)
+        hipLaunchKernelGGL(dev::solveApply<dev::kPassFirstPV>, grid, blkA, 0, stream_, P, it, par);
+      else
+        hipLaunchKernelGGL(dev::solveApply<dev::kPassPV>, grid, blkA, 0, stream_, P, it, par);
+      hipLaunchKernelGGL(dev::solveApply<dev::kPassST>, grid, blkA, 0, stream_, P, it, par ^ 1);
+      if (it == 0)
+        hipLaunchKernelGGL(dev::solveUpdate<true>, grid, blkU, 0, stream_, P, it, par);
+      else
+        hipLaunchKernelGGL(dev::solveUpdate<false>, grid, blkU, 0, stream_, P, it, par);
     }
+    hipLaunchKernelGGL(dev::solveFinish, dim3(1), blkU, 0, stream_, P, n, (3 * (it0 + k)) & 1, flags);
   }
 
   // One full k-omega step.  The collide-stream, the first sub-step's
@@ -2507,13 +2503,13 @@ class EngineT final : public Engine {
       int rc = replay(key, [&] {
         launchLB(options);
         enqueueKoHead(true);
-        enqueueIters(batch);
+        enqueueIters(koSystems(), 2, 0, batch);
       }, 1, err);
       if (rc) return rc;
     } else {
       launchLB(options);
       enqueueKoHead(true);
-      enqueueIters(batch);
+      enqueueIters(koSystems(), 2, 0, batch);
     }
     return koSubSteps(batch, err);
   }
@@ -2538,9 +2534,9 @@ class EngineT final : public Engine {
       HIP_TRY(batchF_.alloc(fBytes));
       HIP_TRY(batchKO_.alloc(6 * D * sizeof(double)));
       HIP_TRY(batchM_.alloc(3 * D * sizeof(R)));
-      HIP_TRY(batchFlags_.alloc(2 * kKoBatch * sizeof(int)));
+      HIP_TRY(batchFlags_.alloc(4 * kKoBatch * sizeof(int)));
       if (!hostFlags_)
-        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&hostFlags_), 2 * kKoBatch * sizeof(int),
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&hostFlags_), 4 * kKoBatch * sizeof(int),
                               hipHostMallocDefault));
     }
     auto copy = [&](void* dst, const void* src, size_t bytes) {
@@ -2575,10 +2571,7 @@ class EngineT final : public Engine {
       for (int i = 0; i < kKoBatch; i++) {
         launchLB(options);
         enqueueKoHead(true);
-        enqueueIters(B);
-        hipLaunchKernelGGL(dev::koBatchFlag, dim3(1), dim3(64), 0, stream_,
-                           (const dev::BicgState*)status_.as<dev::BicgState>(), i,
-                           batchFlags_.as<int>());
+        enqueueIters(koSystems(), 2, 0, B, batchFlags_.as<int>() + 4 * i);
       }
     }, kKoBatch, err);
     if (rc) return rc;
@@ -2586,14 +2579,14 @@ class EngineT final : public Engine {
     // koTimeControl for each step: with one sub-step per LB step only the
     // count of quiet steps changes
     sinceDtChange_ = (sinceDtChange_ + kKoBatch) % kDtQuiet;
-    HIP_TRY(hipMemcpyAsync(hostFlags_, batchFlags_.as<void>(), 2 * kKoBatch * sizeof(int),
+    HIP_TRY(hipMemcpyAsync(hostFlags_, batchFlags_.as<void>(), 4 * kKoBatch * sizeof(int),
                            hipMemcpyDeviceToHost, stream_));
     HIP_TRY(hipStreamSynchronize(stream_));
     bool ok = true;
     int iters = 1;
     for (int i = 0; i < kKoBatch; i++) {
-      ok = ok && hostFlags_[2 * i] == 1;
-      iters = std::max(iters, hostFlags_[2 * i + 1]);
+      ok = ok && hostFlags_[4 * i] && !hostFlags_[4 * i + 1];
+      iters = std::max(iters, hostFlags_[4 * i + 2]);
     }
     if (ok) {
       lastIters_ = iters;
@@ -2618,7 +2611,7 @@ class EngineT final : public Engine {
     koTimeControl();
     const int batch = std::min(std::max(1, lastIters_), 8);
     enqueueKoHead(true);
-    enqueueIters(batch);
+    enqueueIters(koSystems(), 2, 0, batch);
     return koSubSteps(batch, err);
   }
 
@@ -2681,35 +2674,42 @@ class EngineT final : public Engine {
         const std::vector<int64_t> key = {3, batch, stepsPerLB_};
         rc = replay(key, [&] {
           enqueueKoHead(false);
-          enqueueIters(batch);
+          enqueueIters(koSystems(), 2, 0, batch);
         }, 0, err);
         if (rc) return rc;
       } else {
         enqueueKoHead(false);
-        enqueueIters(batch);
+        enqueueIters(koSystems(), 2, 0, batch);
       }
       launched = batch;
     }
   }
 
-  // Polls a solve on the vectors V until both systems are done (adding
-  // chunks of four iterations); lastIters gets the iterations it took.
-  int solveFinish(int launched, const dev::BicgVecs& V, int& lastIters, std::string& err) {
+  // Polls the two systems' solve until both are done (adding chunks of four
+  // iterations).
+  int pollPair(int launched, const dev::SolvePair& P, std::string& err) {
     const int maxIt = std::max(par_.maxIters[0], par_.maxIters[1]);
     int it = launched;
-    auto* st = status_.as<dev::BicgState>();
-    const dev::BicgState& hs = *hostStatus_;
+    const dev::SolveState* hs = hostStatus_;
     while (true) {
-      HIP_TRY(hipMemcpyAsync(hostStatus_, st, sizeof(hs), hipMemcpyDeviceToHost, stream_));
+      HIP_TRY(hipMemcpyAsync(hostStatus_, status_.as<void>(), 2 * sizeof(hs[0]),
+                             hipMemcpyDeviceToHost, stream_));
       HIP_TRY(hipStreamSynchronize(stream_));
-      if ((hs.done[0] && hs.done[1]) || it >= maxIt || hs.nan) break;
+      if (hs[0].nan || hs[1].nan || (hs[0].done && hs[1].done) || it >= maxIt) break;
       const int k = std::min(4, maxIt - it);
-      enqueueIters(k, V);
+      enqueueIters(P, 2, it, k);
       it += k;
     }
-    lastIters = std::max(hs.iters[0], hs.iters[1]);
     HIP_TRY(hipGetLastError());
-    if (hs.nan) {
+    return 0;
+  }
+
+  // The adjoint's transposed systems; lastIters gets the iterations they took.
+  int solveFinish(int launched, const dev::SolvePair& P, int& lastIters, std::string& err) {
+    const int rc = pollPair(launched, P, err);
+    if (rc) return rc;
+    lastIters = std::max(hostStatus_[0].iters, hostStatus_[1].iters);
+    if (hostStatus_[0].nan || hostStatus_[1].nan) {
       err = "non-finite residual in a transposed k-omega solve (the exact tangent of the k-omega "
             "step overflowed; KOFM_ADJOINT_FROZEN_TURBULENCE gives a bounded gradient)";
       return KOFM_ERR_SOLVER_NAN;
@@ -2717,24 +2717,12 @@ class EngineT final : public Engine {
     return 0;
   }
 
-  // Polls the solve until both systems are done (adding chunks of four
-  // iterations); nan reports a non-finite residual.
+  // The k and omega systems; nan reports a non-finite residual.
   int koFinish(int launched, bool& nan, std::string& err) {
-    const int maxIt = std::max(par_.maxIters[0], par_.maxIters[1]);
-    int it = launched;
-    auto* st = status_.as<dev::BicgState>();
-    const dev::BicgState& hs = *hostStatus_;
-    while (true) {
-      HIP_TRY(hipMemcpyAsync(hostStatus_, st, sizeof(hs), hipMemcpyDeviceToHost, stream_));
-      HIP_TRY(hipStreamSynchronize(stream_));
-      if (hs.nan || (hs.done[0] && hs.done[1]) || it >= maxIt) break;
-      const int k = std::min(4, maxIt - it);
-      enqueueIters(k);
-      it += k;
-    }
-    nan = hs.nan != 0;
-    lastIters_ = std::max(hs.iters[0], hs.iters[1]);
-    HIP_TRY(hipGetLastError());
+    const int rc = pollPair(launched, koSystems(), err);
+    if (rc) return rc;
+    nan = hostStatus_[0].nan || hostStatus_[1].nan;
+    lastIters_ = std::max(hostStatus_[0].iters, hostStatus_[1].iters);
     return 0;
   }
 };
@@ -2996,10 +2984,9 @@ class EnsembleT final : public Ensemble {
     std::vector<int> builtParity;
     std::vector<uint64_t> builtGen;  // members' generations when the tables were built
 
-    // k-omega members: the solver states, their gathered flags (pinned on
-    // the host), and the captured steps keyed by the iteration predictions
-    // and the entry parity
-    Buffer koStates, koFlags;
+    // k-omega members: their solves' flags (pinned on the host), and the
+    // captured steps keyed by the iteration predictions and the entry parity
+    Buffer koFlags;
     int* koFlagsHost = nullptr;
     std::vector<std::pair<std::vector<int>, hipGraphExec_t>> koGraphs;
     int koShift = 0;
@@ -3238,15 +3225,10 @@ class EnsembleT final : public Ensemble {
       if (e->stepsPerLB_ != 1)
         return fail(err, "ensemble k-omega members take one k-omega sub-step per LB step "
                          "(ko_dt = 1, time step not halved)");
-    if (g.koStates.bytes() == 0) {
-      std::vector<const dev::BicgState*> ptrs;
-      for (auto* e : g.m) ptrs.push_back(e->status_.template as<dev::BicgState>());
-      HIP_TRY(g.koStates.alloc(ptrs.size() * sizeof(ptrs[0])));
-      HIP_TRY(g.koFlags.alloc(4 * ptrs.size() * sizeof(int)));
-      HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&g.koFlagsHost), 4 * ptrs.size() * sizeof(int),
+    if (g.koFlags.bytes() == 0) {
+      HIP_TRY(g.koFlags.alloc(4 * size_t(nm) * sizeof(int)));
+      HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&g.koFlagsHost), 4 * size_t(nm) * sizeof(int),
                             hipHostMallocDefault));
-      HIP_TRY(hipMemcpy(g.koStates.template as<void>(), ptrs.data(), ptrs.size() * sizeof(ptrs[0]),
-                        hipMemcpyHostToDevice));
     }
     // member k-omega launches go to the ensemble's stream
     struct Swap {
@@ -3265,7 +3247,8 @@ class EnsembleT final : public Ensemble {
     auto solves = [&](const std::vector<int>& batch) {
       for (int i = 0; i < nm; i++) {
         g.m[i]->enqueueKoHead();
-        g.m[i]->enqueueIters(batch[i]);
+        g.m[i]->enqueueIters(g.m[i]->koSystems(), 2, 0, batch[i],
+                             g.koFlags.template as<int>() + 4 * i);
       }
     };
     for (int s = 0; s < n; s++) {
@@ -3320,23 +3303,21 @@ class EnsembleT final : public Ensemble {
       std::vector<int> it(batch);
       const int* flags = g.koFlagsHost;
       while (true) {
-        hipLaunchKernelGGL(dev::bicgGather, dim3((nm + 63) / 64), dim3(64), 0, stream_,
-                           (const dev::BicgState* const*)g.koStates.template as<const dev::BicgState*>(), nm,
-                           g.koFlags.template as<int>());
         HIP_TRY(hipMemcpyAsync(g.koFlagsHost, g.koFlags.template as<void>(), 4 * size_t(nm) * sizeof(int),
                                hipMemcpyDeviceToHost, stream_));
         HIP_TRY(hipStreamSynchronize(stream_));
         bool more = false;
         for (int i = 0; i < nm; i++) {
-          if (flags[4 * i + 3]) {
+          if (flags[4 * i + 1]) {
             err = "non-finite residual in the k-omega solve of an ensemble member";
             return KOFM_ERR_SOLVER_NAN;
           }
           const EngineT<S, R>* e = g.m[i];
           const int maxIt = std::max(e->par_.maxIters[0], e->par_.maxIters[1]);
-          if (!(flags[4 * i] && flags[4 * i + 1]) && it[i] < maxIt) {
+          if (!flags[4 * i] && it[i] < maxIt) {
             const int k = std::min(4, maxIt - it[i]);
-            g.m[i]->enqueueIters(k);
+            g.m[i]->enqueueIters(g.m[i]->koSystems(), 2, it[i], k,
+                                 g.koFlags.template as<int>() + 4 * i);
             it[i] += k;
             more = true;
           }

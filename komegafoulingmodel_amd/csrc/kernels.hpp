@@ -1183,278 +1183,11 @@ __device__ __forceinline__ void koCoeffRow(
   o.bo = out[ko::kRowBo];
 }
 
-// ---------------------------------------------------------------------------
-// implicit k / omega solve: BiCGStab for both systems at once
-// ---------------------------------------------------------------------------
-//
-// The assembled rows (diagonal 1, four neighbours) are not diagonally
-// dominant next to curved walls, so a stationary iteration can diverge; the
-// reference uses restarted GMRES (GMRESSolver.cpp:227-355).  Here both systems
-// run unpreconditioned BiCGStab (van der Vorst 1992) in lock step, iterating
-// in place on K and O: three streaming kernels per iteration with the
-// neighbour values of p and s recomputed in registers (so p, v are double-
-// buffered and s needs no separate pass), each followed by a one-block
-// kernel that turns the per-block FP64 partial dot products into the
-// scalars.  The streaming kernels run a fixed number of blocks that walk
-// their XCD's band of row tiles, so there are few partials to sum.  The
-// first residual r = b - A x is formed by the coefficient kernel itself.
-// All scalars stay in device memory; the host only polls the done flags.
-// (Cross-block reduction inside one kernel would need agent-scope release
-// fences, which write back the L2 and cost far more than a launch here.)
-
-struct BicgState {
-  double rho[2], rhoNew[2], alpha[2], omega[2], beta[2];
-  double r0[2], rn[2];
-  double rtol[2], atol[2];
-  double best[2];   // smallest residual so far
-  double bnorm[2];  // ||b|| (stopping rule 1)
-  double prevRes[2];  // the previous iteration's residual (stopping rule 1)
-  int crit[2];      // stopping rule: 0 as GMRESSolver, 1 as BiCGStabSolver
-  int maxit[2];
-  int done[2];
-  int iters[2];
-  int restart[2];
-  int sinceBest[2]; // iterations since the residual last fell below 0.999 best
-  int nan;
-  int cur;  // which p/v buffer holds the current iterate
-};
-
-// A solve whose residual has not fallen below 0.999 of its best for this
-// many iterations has reached the rounding floor of FP64 and stops: past
-// that point the recursively updated residual no longer follows b - A x,
-// and further iterations move x without improving it.
-constexpr int kBicgStagnation = 50;
-
-// Solver vectors are FP64 for every storage form: the omega field spans about
-// seven decades (wall rows near 1000, core values near 1e-4) and FP32 Krylov
-// vectors cannot resolve the core next to the wall.
-struct BicgVecs {
-  double* x[2];        // K, O in HBM (the iterate)
-  double* A[2];        // 4 planes each: E, W, N, S
-  double* b[2];
-  double* r[2];
-  double* rh[2];
-  double* p[2][2];     // [variable][buffer]
-  double* v[2][2];
-  double* s[2];
-  double* t[2];
-  double* partial;     // 4 doubles per block
-  double* prev[2];     // when set, koCoeffs keeps the initial K, O here (restart point)
-};
-
 __device__ __forceinline__ void nbIndex(const KOParams& p, int x, size_t g, size_t (&nb)[4]) {
   nb[0] = x < p.nX - 1 ? g + 1 : g - x;        // E
   nb[1] = x > 0 ? g - 1 : g + (p.nX - 1);      // W
   nb[2] = g + p.XF;                            // N
   nb[3] = g - p.XF;                            // S
-}
-
-// Calls f(x, y) for every node of the row tiles this block owns: the
-// blocks of XCD k = blockIdx % 8 walk the k-th band of tiles (so a stencil's
-// neighbour rows stay in that XCD's L2) with a stride of gridDim / 8.
-template <class F>
-__device__ __forceinline__ void forOwnTiles(const KOParams& p, F&& f) {
-  const int xcd = int(blockIdx.x & 7), stride = int(gridDim.x >> 3);
-  const int end = min((xcd + 1) * p.tiles.per, p.tiles.nTiles);
-  for (int T = xcd * p.tiles.per + int(blockIdx.x >> 3); T < end; T += stride) {
-    const int x = (T % p.tiles.tilesX) * kBlockX + int(threadIdx.x);
-    if (x < p.nX) f(x, T / p.tiles.tilesX);
-  }
-}
-
-// per-block sums of two doubles per variable -> partial[blk*4 + v*2 + k]
-__device__ __forceinline__ void blockPartials(double (&a)[2][2], double* __restrict__ partial) {
-  __shared__ double red[2][2][kBlockX / 64];
-#pragma unroll
-  for (int v = 0; v < 2; v++)
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-      double x = a[v][k];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-      if ((threadIdx.x & 63) == 0) red[v][k][threadIdx.x >> 6] = x;
-    }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    const int v = threadIdx.x >> 1, k = threadIdx.x & 1;
-    double sum = 0.;
-#pragma unroll
-    for (int w = 0; w < kBlockX / 64; w++) sum += red[v][k][w];
-    partial[size_t(blockIdx.x) * 4 + threadIdx.x] = sum;
-  }
-}
-
-__device__ __forceinline__ void sumPartials(const double* __restrict__ partial, int nblk,
-                                            double (&out)[4]) {
-  __shared__ double red[4][16];
-  double a[4] = {0., 0., 0., 0.};
-  for (int i = threadIdx.x; i < nblk; i += blockDim.x)
-#pragma unroll
-    for (int k = 0; k < 4; k++) a[k] += partial[size_t(i) * 4 + k];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) a[k] += __shfl_xor(a[k], off, 64);
-    if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = a[k];
-  }
-  __syncthreads();
-  for (int k = 0; k < 4; k++) {
-    double s = 0.;
-    for (int w = 0; w < int(blockDim.x + 63) / 64; w++) s += red[k][w];
-    out[k] = s;
-  }
-}
-
-// Scalar updates between the streaming kernels (one block of 1024 threads).
-// stage 0: after the coefficients (r0), 1: after bicgPV (alpha), 2: after
-// bicgST (omega), 3: after bicgXR (rho, beta, convergence).
-__global__ __launch_bounds__(1024) void bicgScalars(const double* __restrict__ partial, int nblk,
-                                                    BicgState* __restrict__ st, int stage) {
-  if (st->done[0] && st->done[1]) return;
-  double s[4];
-  sumPartials(partial, nblk, s);
-  if (threadIdx.x != 0) return;
-  for (int v = 0; v < 2; v++) {
-    if (st->done[v]) continue;
-    const double a = s[2 * v], b = s[2 * v + 1];
-    if (stage == 0) {
-      // a = (r, r), b = (b, b) (rule 1); the first bicgPV takes p = r
-      // (restart form), rh = r
-      const double r0 = sqrt(a);
-      st->r0[v] = r0;
-      st->rn[v] = r0;
-      st->iters[v] = 0;
-      st->rho[v] = st->alpha[v] = st->omega[v] = 1.;
-      st->rhoNew[v] = a;
-      st->beta[v] = a;
-      st->restart[v] = 1;
-      st->best[v] = r0;
-      st->sinceBest[v] = 0;
-      st->prevRes[v] = r0;
-      if (st->crit[v] == 1) {
-        // BiCGStabSolver::solve (BiCGStabSolver.cpp:648-658): ||b|| <= 1e-16
-        // ends the solve (the kernel leaves x; the reference copies b, the
-        // same zero field up to 1e-16)
-        const double bn = sqrt(b);
-        st->bnorm[v] = bn;
-        if (!isfinite(r0) || !isfinite(bn)) {
-          st->nan = 1;
-          st->done[v] = 1;
-        } else if (bn <= 1.0e-16 || r0 == 0. || r0 <= st->rtol[v] * bn) {
-          st->done[v] = 1;
-        }
-      } else if (!isfinite(r0)) {
-        st->nan = 1;
-        st->done[v] = 1;
-      } else if (r0 == 0. || r0 <= st->atol[v]) {
-        st->done[v] = 1;
-      }
-    } else if (stage == 1) {
-      // a = (rh, v); a restart requested by the last stage 3 has now been
-      // consumed by bicgPV
-      st->restart[v] = 0;
-      if (a == 0. || !isfinite(a)) {
-        st->alpha[v] = 0.;
-        st->restart[v] = 1;
-      } else {
-        st->alpha[v] = st->rhoNew[v] / a;
-      }
-    } else if (stage == 2) {
-      // a = (t, s), b = (t, t)
-      st->omega[v] = (b > 0. && isfinite(b)) ? a / b : 0.;
-    } else {
-      // a = (rh, r), b = (r, r)
-      const double rn = sqrt(b);
-      st->iters[v] += 1;
-      st->rn[v] = rn;
-      if (!isfinite(rn)) {
-        st->nan = 1;
-        st->done[v] = 1;
-        continue;
-      }
-      if (st->crit[v] == 1) {
-        // BiCGStabSolver::reduceAndCheckConvergence (BiCGStabSolver.cpp:509-545):
-        // a residual above 10 times the last one after the first iteration
-        // fails like a non-finite one (the caller halves the time step);
-        // converged at ||r|| <= rtol ||b|| or ||r|| <= atol ||r0||
-        if (st->iters[v] > 1 && rn > 10. * st->prevRes[v]) {
-          st->nan = 1;
-          st->done[v] = 1;
-          continue;
-        }
-        st->prevRes[v] = rn;
-        if (rn <= st->rtol[v] * st->bnorm[v] || rn <= st->atol[v] * st->r0[v] ||
-            st->iters[v] >= st->maxit[v]) {
-          st->done[v] = 1;
-          continue;
-        }
-      } else if (rn <= st->rtol[v] * st->r0[v] || rn <= st->atol[v] ||
-                 st->iters[v] >= st->maxit[v]) {
-        st->done[v] = 1;
-        continue;
-      }
-      if (rn < 0.999 * st->best[v]) {
-        st->best[v] = rn;
-        st->sinceBest[v] = 0;
-      } else if (++st->sinceBest[v] >= kBicgStagnation) {
-        st->done[v] = 1;
-        continue;
-      }
-      st->rho[v] = st->rhoNew[v];
-      st->rhoNew[v] = a;
-      if (a == 0. || st->omega[v] == 0. || st->restart[v]) {
-        // breakdown or stagnation: restart with rh = r, p = v = 0
-        st->restart[v] = 1;
-        st->rho[v] = st->alpha[v] = st->omega[v] = 1.;
-        st->rhoNew[v] = b;
-        st->beta[v] = b;
-      } else {
-        st->beta[v] = (a / st->rho[v]) * (st->alpha[v] / st->omega[v]);
-      }
-    }
-  }
-  if (stage == 3) st->cur ^= 1;
-}
-
-// Update_kOmega_Coeffs_Implicit (kOmegaKernels.cl:187-480): the normalised
-// rows of both systems, then the first residual r = b - A x from the current
-// K and O (the solve's initial guess); partials (r, r).
-template <class M>
-__global__ __launch_bounds__(kBlockX) void koCoeffs(
-    const uint16_t* __restrict__ mask, const double* __restrict__ Nut, const double* __restrict__ Dk,
-    const double* __restrict__ Do, const double* __restrict__ F1a, const double* __restrict__ dkdo,
-    const double* __restrict__ Sx, const M* __restrict__ rho, const M* __restrict__ uxa,
-    const M* __restrict__ uya, const double* __restrict__ dX, const double* __restrict__ Wd,
-    BicgVecs V, KOParams p) {
-  double a[2][2] = {{0., 0.}, {0., 0.}};
-  forOwnTiles(p, [&](int x, int y) {
-    const size_t g = size_t(x) + size_t(p.XF) * y;
-    const uint32_t m = mask[g];
-    if (m & kSolid) return;
-    const double* K = V.x[0];
-    const double* O = V.x[1];
-    KORows o;
-    koCoeffRow<M>(x, g, m, K, O, Nut, Dk, Do, F1a, dkdo, Sx, rho, uxa, uya, dX, Wd, p, o);
-    size_t nb[4];
-    nbIndex(p, x, g, nb);
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-      const double* A = v == 0 ? o.Ak : o.Ao;
-      const double* X = V.x[v];
-      if (V.prev[v]) V.prev[v][g] = X[g];
-#pragma unroll
-      for (int d = 0; d < 4; d++) V.A[v][g + size_t(d) * p.D] = A[d];
-      const double b = v == 0 ? o.bk : o.bo;
-      V.b[v][g] = b;
-      const double ax = X[g] + (A[0] * X[nb[0]] + A[1] * X[nb[1]] + A[2] * X[nb[2]] +
-                                A[3] * X[nb[3]]);
-      const double r = b - ax;
-      V.r[v][g] = r;
-      V.rh[v][g] = r;
-      a[v][0] += r * r;
-    }
-  });
-  blockPartials(a, V.partial);
 }
 
 // K, O of every non-solid node back from the copies koCoeffs kept at the
@@ -1500,263 +1233,6 @@ __global__ __launch_bounds__(kBlockX) void solverPairs(uint16_t* __restrict__ ma
       m |= kPairUp;  // the one before it
   }
   mask[i] = uint16_t(m);
-}
-
-// (M^-1 u)_i for u given by a function of the node index: with partner q,
-// (u_i - a_iq u_q) / (1 - a_iq a_qi), the couplings taken from the rows in
-// A (for a transposed system A holds the transposed rows, so this is M^T).
-template <class F>
-__device__ __forceinline__ double pairSolve(uint32_t m, const double* __restrict__ A, size_t i,
-                                            const KOParams& p, F u) {
-  if (!(m & (kPairUp | kPairDown))) return u(i);
-  const bool up = (m & kPairUp) != 0;
-  const size_t q = up ? i + size_t(p.XF) : i - size_t(p.XF);
-  const double aiq = A[i + size_t(up ? 2 : 3) * p.D];
-  const double aqi = A[q + size_t(up ? 3 : 2) * p.D];
-  return (u(i) - aiq * u(q)) / (1. - aiq * aqi);
-}
-
-// Right-preconditioned BiCGStab (van der Vorst 1992, Algorithm with M on the
-// right): p' = r + beta (p - omega v), v' = A M^-1 p' (neighbour values
-// recomputed); partials (rh, v').  On a restart p' = r and rh is reset to r.
-__global__ __launch_bounds__(kBlockX) void bicgPV(const uint16_t* __restrict__ mask, BicgVecs V,
-                                                  const BicgState* __restrict__ st, KOParams p) {
-  if (st->done[0] && st->done[1]) return;
-  const int cur = st->cur;
-  double a[2][2] = {{0., 0.}, {0., 0.}};
-  forOwnTiles(p, [&](int x, int y) {
-    const size_t g = size_t(x) + size_t(p.XF) * y;
-    if (mask[g] & kSolid) return;
-    size_t nb[4];
-    nbIndex(p, x, g, nb);
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-      if (st->done[v]) continue;
-      const double* r = V.r[v];
-      const double* po = V.p[v][cur];
-      const double* vo = V.v[v][cur];
-      const double* A = V.A[v];
-      const bool rs = st->restart[v] != 0;
-      const double beta = st->beta[v], om = st->omega[v];
-      auto pn = [&](size_t i) { return rs ? r[i] : r[i] + beta * (po[i] - om * vo[i]); };
-      auto ph = [&](size_t i) { return pairSolve(mask[i], A, i, p, pn); };
-      const double pc = pn(g);
-      const double vc = ph(g) + (A[g] * ph(nb[0]) + A[g + p.D] * ph(nb[1]) +
-                                 A[g + 2 * p.D] * ph(nb[2]) + A[g + 3 * p.D] * ph(nb[3]));
-      V.p[v][cur ^ 1][g] = pc;
-      V.v[v][cur ^ 1][g] = vc;
-      double rh = V.rh[v][g];
-      if (rs) {
-        rh = r[g];
-        V.rh[v][g] = rh;
-      }
-      a[v][0] += rh * vc;
-    }
-  });
-  blockPartials(a, V.partial);
-}
-
-// s = r - alpha v' (neighbours recomputed), t = A M^-1 s; partials (t, s), (t, t).
-__global__ __launch_bounds__(kBlockX) void bicgST(const uint16_t* __restrict__ mask, BicgVecs V,
-                                                  const BicgState* __restrict__ st, KOParams p) {
-  if (st->done[0] && st->done[1]) return;
-  const int nxt = st->cur ^ 1;
-  double a[2][2] = {{0., 0.}, {0., 0.}};
-  forOwnTiles(p, [&](int x, int y) {
-    const size_t g = size_t(x) + size_t(p.XF) * y;
-    if (mask[g] & kSolid) return;
-    size_t nb[4];
-    nbIndex(p, x, g, nb);
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-      if (st->done[v]) continue;
-      const double* r = V.r[v];
-      const double* vv = V.v[v][nxt];
-      const double* A = V.A[v];
-      const double al = st->alpha[v];
-      auto sn = [&](size_t i) { return r[i] - al * vv[i]; };
-      auto sh = [&](size_t i) { return pairSolve(mask[i], A, i, p, sn); };
-      const double sc = sn(g);
-      const double tc = sh(g) + (A[g] * sh(nb[0]) + A[g + p.D] * sh(nb[1]) +
-                                 A[g + 2 * p.D] * sh(nb[2]) + A[g + 3 * p.D] * sh(nb[3]));
-      V.s[v][g] = sc;
-      V.t[v][g] = tc;
-      a[v][0] += tc * sc;
-      a[v][1] += tc * tc;
-    }
-  });
-  blockPartials(a, V.partial);
-}
-
-// x += alpha M^-1 p' + omega M^-1 s, r = s - omega t; partials (rh, r), (r, r).
-__global__ __launch_bounds__(kBlockX) void bicgXR(const uint16_t* __restrict__ mask, BicgVecs V,
-                                                  const BicgState* __restrict__ st, KOParams p) {
-  if (st->done[0] && st->done[1]) return;
-  const int nxt = st->cur ^ 1;
-  double a[2][2] = {{0., 0.}, {0., 0.}};
-  forOwnTiles(p, [&](int x, int y) {
-    const size_t g = size_t(x) + size_t(p.XF) * y;
-    const uint32_t m = mask[g];
-    if (m & kSolid) return;
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-      if (st->done[v]) continue;
-      const double al = st->alpha[v], om = st->omega[v];
-      const double* pv = V.p[v][nxt];
-      const double* sv = V.s[v];
-      const double sc = sv[g];
-      const double ph = pairSolve(m, V.A[v], g, p, [&](size_t i) { return pv[i]; });
-      const double sh = pairSolve(m, V.A[v], g, p, [&](size_t i) { return sv[i]; });
-      V.x[v][g] += al * ph + om * sh;
-      const double r = sc - om * V.t[v][g];
-      V.r[v][g] = r;
-      a[v][0] += V.rh[v][g] * r;
-      a[v][1] += r * r;
-    }
-  });
-  blockPartials(a, V.partial);
-}
-
-// Step i of a batch of k-omega steps: out[2 i] = 1 when both solves have
-// finished with finite residuals, out[2 i + 1] = the iterations they took.
-__global__ void koBatchFlag(const BicgState* __restrict__ st, int i, int* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  out[2 * i] = (st->done[0] && st->done[1] && !st->nan) ? 1 : 0;
-  out[2 * i + 1] = st->iters[0] > st->iters[1] ? st->iters[0] : st->iters[1];
-}
-
-// Done flags, iteration count and NaN flag of several solver states (an
-// ensemble's members) in one array: out[4 i .. 4 i + 3].
-__global__ void bicgGather(const BicgState* const* __restrict__ st, int n, int* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const BicgState* s = st[i];
-  out[4 * i] = s->done[0];
-  out[4 * i + 1] = s->done[1];
-  out[4 * i + 2] = s->iters[0] > s->iters[1] ? s->iters[0] : s->iters[1];
-  out[4 * i + 3] = s->nan;
-}
-
-// Resets the solver state for a new solve (a kernel, not a memset, so the
-// step can be captured into a graph).
-__global__ void bicgReset(BicgState* __restrict__ st, double relK, double absK, int maxK,
-                          double relO, double absO, int maxO) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  BicgState z = {};
-  z.rtol[0] = relK;
-  z.atol[0] = absK;
-  z.maxit[0] = maxK;
-  z.rtol[1] = relO;
-  z.atol[1] = absO;
-  z.maxit[1] = maxO;
-  *st = z;
-}
-
-// The solver state for the temperature system: system 0 with
-// BiCGStabSolver's stopping rule, system 1 empty (its partials are zero, so
-// it is done at stage 0).
-__global__ void bicgResetT(BicgState* __restrict__ st, double rel, double abs_, int maxit) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  BicgState z = {};
-  z.rtol[0] = rel;
-  z.atol[0] = abs_;
-  z.maxit[0] = maxit;
-  z.crit[0] = 1;
-  *st = z;
-}
-
-// ---------------------------------------------------------------------------
-// temperature (clVariablesFD)
-// ---------------------------------------------------------------------------
-
-struct TParams {
-  double alphaFluid, alphaFoul, prTurbInv, tIn;
-};
-
-// The three-point weights of Update_T_Coeffs_Implicit (tfdKernels.cl:154-181):
-// spacings held at 0.1 or more; the first derivative falls back to the
-// two-point central difference where |the tested weight| > 10 (the x row
-// tests its centre weight, the y row its north weight, as the kernel does).
-__device__ __forceinline__ void tWeights(double dp, double dm, bool testCentre, double (&d1)[3],
-                                         double (&d2)[3]) {
-  dp = fmax(dp, 0.1);
-  dm = fmax(dm, 0.1);
-  const double dc = fmax(dp + dm, 0.1);
-  d1[0] = dm / (dp * dc);
-  d1[1] = -dp / (dm * dc);
-  d1[2] = (dp - dm) / (dp * dm);
-  d2[0] = 2. / (dp * dc);
-  d2[1] = 2. / (dm * dc);
-  d2[2] = -2. / (dp * dm);
-  if (fabs(testCentre ? d1[2] : d1[0]) > 10.) {
-    d1[0] = 1. / dc;
-    d1[1] = -1. / dc;
-    d1[2] = 0.;
-  }
-}
-
-// Update_T_Coeffs_Implicit (tfdKernels.cl:122-280) in the five-point row
-// form of the k-omega systems (diagonal 1; planes E, W, N, S), then the first
-// residual r = b - A T from the current T; partials (r, r) and (b, b) of
-// system 0 (system 1 gets zeros).  Rows on the nodes of tmask that are not
-// solid (solid in the clean geometry); a node solid in the LB mask (the
-// fouling layer) takes alphaFoul.  nu_t / Pr_t adds to alpha and the x and y
-// differences of nu_t to the advection (the kernel multiplies the centre
-// term by 1 / Pr_t twice, which is kept).  The source is T clamped to
-// [0, T_in]; the inlet column's W coefficient moves to the right-hand side
-// with T_in and the outlet column's E coefficient into the diagonal.  When
-// Tprev is set, T is also copied there (the restart point of the step).
-template <class M>
-__global__ __launch_bounds__(kBlockX) void thermalCoeffs(
-    const uint16_t* __restrict__ tmask, const uint16_t* __restrict__ lbmask,
-    const double* __restrict__ dX0, const double* __restrict__ Nut, const M* __restrict__ uxa,
-    const M* __restrict__ uya, double* __restrict__ Tprev, BicgVecs V, TParams tp, double dt,
-    KOParams p) {
-  double a[2][2] = {{0., 0.}, {0., 0.}};
-  forOwnTiles(p, [&](int x, int y) {
-    const size_t g = size_t(x) + size_t(p.XF) * y;
-    if (tmask[g] & kSolid) return;
-    const double* T = V.x[0];
-    double dx1[3], dx2[3], dy1[3], dy2[3];
-    tWeights(dX0[g], dX0[g + p.D], true, dx1, dx2);
-    tWeights(dX0[g + 2 * p.D], dX0[g + 3 * p.D], false, dy1, dy2);
-    size_t nb[4];
-    nbIndex(p, x, g, nb);
-    double alpha = (lbmask[g] & kSolid) ? tp.alphaFoul : tp.alphaFluid;
-    const double at = Nut[g] * tp.prTurbInv;
-    const double Jx = double(uxa[g]) -
-                      tp.prTurbInv * (dx1[0] * Nut[nb[0]] + dx1[1] * Nut[nb[1]] + dx1[2] * at);
-    const double Jy = double(uya[g]) -
-                      tp.prTurbInv * (dy1[0] * Nut[nb[2]] + dy1[1] * Nut[nb[3]] + dy1[2] * at);
-    alpha += at;
-    const double Tg = T[g];
-    double src = fmin(fmax(0., Tg), tp.tIn);
-    double C = 1. + dt * (Jx * dx1[2] + Jy * dy1[2] - alpha * (dx2[2] + dy2[2]));
-    const double S = dt * (Jy * dy1[1] - alpha * dy2[1]);
-    const double W = dt * (Jx * dx1[1] - alpha * dx2[1]);
-    if (x == 0) src -= tp.tIn * W;
-    const double E = dt * (Jx * dx1[0] - alpha * dx2[0]);
-    if (x == p.nX - 1) C += E;
-    const double N = dt * (Jy * dy1[0] - alpha * dy2[0]);
-    const double inv = 1. / C;
-    double A[4];
-    A[0] = x < p.nX - 1 ? E * inv : 0.;
-    A[1] = x > 0 ? W * inv : 0.;
-    A[2] = N * inv;
-    A[3] = S * inv;
-    const double b = src * inv;
-#pragma unroll
-    for (int d = 0; d < 4; d++) V.A[0][g + size_t(d) * p.D] = A[d];
-    V.b[0][g] = b;
-    const double ax = Tg + (A[0] * T[nb[0]] + A[1] * T[nb[1]] + A[2] * T[nb[2]] + A[3] * T[nb[3]]);
-    const double r = b - ax;
-    V.r[0][g] = r;
-    V.rh[0][g] = r;
-    if (Tprev) Tprev[g] = Tg;
-    a[0][0] += r * r;
-    a[0][1] += b * b;
-  });
-  blockPartials(a, V.partial);
 }
 
 // ---------------------------------------------------------------------------

@@ -562,12 +562,11 @@ __global__ __launch_bounds__(kBlockX) void koTranspose(const uint16_t* __restric
 }
 
 // r = b - A x of both systems; sums (r, r).
-__global__ __launch_bounds__(kStripX) void solveResidual(SolvePair P, const double* __restrict__ bk,
-                                                         const double* __restrict__ bo, KOParams p) {
-  Chunk c;
-  if (!chunkOf(P.sys[0].s, p.nX, p.nY, c)) return;
+__global__ __launch_bounds__(kTileLanes) void solveResidual(SolvePair P, const double* __restrict__ bk,
+                                                            const double* __restrict__ bo, KOParams p,
+                                                            Tiles tiles) {
   Sum acc[2]{};
-  forChunk(c, [&](int x, int y) {
+  forTileNodes(tiles, p.nX, p.nY, [&](int x, int y) {
     const size_t g = size_t(x) + size_t(p.XF) * y;
     if (P.sys[0].mask[g] & kSolid) return;
     size_t nb[4];
@@ -583,8 +582,8 @@ __global__ __launch_bounds__(kStripX) void solveResidual(SolvePair P, const doub
       acc[v].add(r * r);
     }
   });
-  writePartial<kStripX>(P.sys[0], c.T, 0, acc[0], Sum{});
-  writePartial<kStripX>(P.sys[1], c.T, 0, acc[1], Sum{});
+  writePartial<kTileLanes>(P.sys[0], int(blockIdx.x), 0, acc[0], Sum{});
+  writePartial<kTileLanes>(P.sys[1], int(blockIdx.x), 0, acc[1], Sum{});
 }
 
 // Step 2: adjoint of the row assembly.

@@ -141,8 +141,9 @@ class EngineT final : public Engine {
     if (ko_)
       for (Buffer* b : solverBuffers()) HIP_TRY(b->alloc(D * sizeof(double)));
     strips_ = dev::stripsFor(nX_, nY_);
+    tiles_ = dev::tilesFor(nX_, nY_);
     // [system][pass parity][block][2] sums, and the pass states behind them
-    HIP_TRY(partial_.alloc(8 * size_t(strips_.nblk) * sizeof(double2)));
+    HIP_TRY(partial_.alloc(8 * size_t(std::max(strips_.nblk, tiles_.blocks)) * sizeof(double2)));
     HIP_TRY(passState_.alloc(4 * sizeof(dev::SolveState)));
     HIP_TRY(redPartial_.alloc(dev::kReducePartials * sizeof(double)));
     HIP_TRY(redOut_.alloc(sizeof(double)));
@@ -228,9 +229,17 @@ class EngineT final : public Engine {
       HIP_TRY(upload<double>(dX_, g.dX));
       HIP_TRY(dX0_.alloc(4 * D * sizeof(double)));
       HIP_TRY(hipMemcpy(dX0_.as<void>(), dX_.as<void>(), 4 * D * sizeof(double), hipMemcpyDeviceToDevice));
+      markUnitSpacing(mask_, dX_);
+      HIP_TRY(hipGetLastError());
     }
     haveGeo_ = true;
     return 0;
+  }
+
+  void markUnitSpacing(const Buffer& mask, const Buffer& dX) {
+    hipLaunchKernelGGL(dev::unitSpacing, dim3(unsigned((D_ + dev::kBlockX - 1) / dev::kBlockX)),
+                       dim3(dev::kBlockX), 0, stream_, mask.as<uint16_t>(),
+                       (const double*)dX.as<double>(), D_);
   }
 
   // Wall-shear tables of geo_ to the device.
@@ -342,6 +351,7 @@ class EngineT final : public Engine {
     hipLaunchKernelGGL(dev::solverPairs, flat, dim3(dev::kBlockX), 0, stream_, mask_.as<uint16_t>(),
                        nX_, XF_, nY_);
     if (ko_) {
+      markUnitSpacing(mask_, dX_);
       HIP_TRY(lsm.alloc(geo_.lsMap.size() * sizeof(uint16_t)));
       HIP_TRY(hipMemcpy(lsm.as<void>(), geo_.lsMap.data(), geo_.lsMap.size() * sizeof(uint16_t),
                         hipMemcpyHostToDevice));
@@ -790,6 +800,7 @@ class EngineT final : public Engine {
     HIP_TRY(hipMemcpy(tmask_.as<void>(), m.data(), D * sizeof(uint16_t), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(dev::solverPairs, dim3(unsigned((D_ + dev::kBlockX - 1) / dev::kBlockX)),
                        dim3(dev::kBlockX), 0, stream_, tmask_.as<uint16_t>(), nX_, XF_, nY_);
+    markUnitSpacing(tmask_, dX0_);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(T_.as<void>(), T.data(), D * sizeof(double), hipMemcpyHostToDevice));
     HIP_TRY(hipStreamSynchronize(stream_));
@@ -838,11 +849,11 @@ class EngineT final : public Engine {
       bool first = true;
       int sub = 0;
       while (sub < tSteps_) {
-        hipLaunchKernelGGL((dev::thermalCoeffs<R>), solveGrid(1), dim3(dev::kStripX), 0, stream_,
+        hipLaunchKernelGGL((dev::thermalCoeffs<R>), dim3(tiles_.blocks), dim3(dev::kTileLanes), 0, stream_,
                            (const uint16_t*)mask_.as<uint16_t>(), (const double*)dX0_.as<double>(),
                            (const double*)nut_.as<double>(), (const R*)ux_.as<R>(),
                            (const R*)uy_.as<R>(), first ? Tprev_.as<double>() : nullptr, P, tpar_,
-                           tDt_, kp);
+                           tDt_, kp, tiles_);
         const int batch = std::min(std::max(1, tIters_), 8);
         enqueueIters(P, 1, 0, batch);
         bool nan = false;
@@ -1206,6 +1217,7 @@ class EngineT final : public Engine {
   Buffer ss_, cfss_, tau_, sInd_, wts_, tauBL_;
   Buffer status_, passState_, partial_, redPartial_, redOut_;
   dev::Strips strips_{};  // the solver passes' blocks
+  dev::Tiles tiles_{};    // the assembly kernels' blocks
   int lastIters_ = 1;  // iterations the previous k-omega solve needed
   // k-omega time step control (kOmega.cpp:31-73, 387-414): sub-steps per LB
   // step, their time step, steps since the last change, and non-finite
@@ -1532,7 +1544,7 @@ class EngineT final : public Engine {
       p.applyIbb = m == 0 ? ap0 : 1;
       launchLBBlock<true>(lbBlock_, lbNpt_, p, seg_[m]->template as<S>(), seg_[m + 1]->template as<S>());
       const int batch = std::min(std::max(1, lastIters_), 8);
-      enqueueKoHead();
+      enqueueKoHead(false, true, true);
       enqueueIters(koSystems(), 2, 0, batch);
       bool nan = false;
       int rc = koFinish(batch, nan, err);
@@ -1556,8 +1568,8 @@ class EngineT final : public Engine {
         // 1. the transposed implicit systems, warm-started from the last solution
         hipLaunchKernelGGL(dev::koTranspose, grid, blk, 0, stream_, mask, (const double*)tapePlane(m, kTAk),
                            (const double*)tapePlane(m, kTAo), adjPlane(kATk), adjPlane(kATo), kp);
-        hipLaunchKernelGGL(dev::solveResidual, solveGrid(1), dim3(dev::kStripX), 0, stream_, P,
-                           (const double*)adjPlane(kAKb), (const double*)adjPlane(kAOb), kp);
+        hipLaunchKernelGGL(dev::solveResidual, dim3(tiles_.blocks), dim3(dev::kTileLanes), 0, stream_, P,
+                           (const double*)adjPlane(kAKb), (const double*)adjPlane(kAOb), kp, tiles_);
         const int batch = std::min(std::max(1, adjIters_), 8);
         enqueueIters(P, 2, 0, batch);
         int rc = solveFinish(batch, P, adjIters_, err);
@@ -2264,7 +2276,8 @@ class EngineT final : public Engine {
     dev::SolveSys y{};
     y.mask = mask_.as<uint16_t>();
     y.st = passState_.as<dev::SolveState>() + 2 * v;
-    y.partial = partial_.as<double2>() + size_t(v) * 4 * strips_.nblk;
+    y.n0 = tiles_.blocks;
+    y.partial = partial_.as<double2>() + size_t(v) * 4 * std::max(strips_.nblk, tiles_.blocks);
     y.nX = nX_;
     y.nY = nY_;
     y.XF = XF_;
@@ -2450,22 +2463,37 @@ class EngineT final : public Engine {
   // the solver passes of n systems
   dim3 solveGrid(int n) const { return dim3(unsigned(8 * strips_.per), unsigned(n)); }
 
-  // kOmega::Solve (kOmega.cpp:31-73), first part: diffusivities, then the
-  // coefficients with the first residual and the solver's stage 0.  The
-  // first sub-step of a step also keeps k and omega as the restart point
-  // (copyToPrevSolution).
-  void enqueueKoHead(bool savePrev = false) {
-    auto kp = koParams();
-    const dim3 grid(8 * kp.tiles.per), blk(dev::kBlockX);
+  // kOmega::Solve (kOmega.cpp:31-73), first part: diffusivities and
+  // coefficients with the first residual.  The first sub-step of a step also
+  // keeps k and omega as the restart point (copyToPrevSolution).  The
+  // diffusivity fields are written unless a later step of the same call
+  // overwrites them, F1 and m grad k for the adjoint's tape only.
+  void enqueueKoHead(bool savePrev = false, bool keepD = true, bool tape = false) {
     using K = double;
-    hipLaunchKernelGGL((dev::koDiffusivities<R>), grid, blk, 0, stream_, mask_.as<uint16_t>(),
-                       K_.as<K>(), O_.as<K>(), nut_.as<K>(), wallD_.as<K>(), Dk_.as<K>(),
-                       Do_.as<K>(), F1_.as<K>(), dkdo_.as<K>(), rho_.as<R>(), dX_.as<K>(), kp);
-    hipLaunchKernelGGL((dev::koCoeffs<R>), solveGrid(1), dim3(dev::kStripX), 0, stream_,
-                       nut_.as<K>(), Dk_.as<K>(), Do_.as<K>(), F1_.as<K>(), dkdo_.as<K>(),
-                       S_.as<K>(), rho_.as<R>(), ux_.as<R>(), uy_.as<R>(), dX_.as<K>(),
-                       wallD_.as<K>(), savePrev ? Kprev_.as<K>() : nullptr,
-                       savePrev ? Oprev_.as<K>() : nullptr, koSystems(), kp);
+    dev::KOAssembly q{};
+    q.nut = nut_.as<K>();
+    q.S = S_.as<K>();
+    q.dX = dX_.as<K>();
+    q.wd = wallD_.as<K>();
+    q.rho = rho_.as<void>();
+    q.ux = ux_.as<void>();
+    q.uy = uy_.as<void>();
+    q.Dk = Dk_.as<K>();
+    q.Do = Do_.as<K>();
+    if (tape) {
+      q.F1 = F1_.as<K>();
+      q.dkdo = dkdo_.as<K>();
+    }
+    if (savePrev) {
+      q.prevK = Kprev_.as<K>();
+      q.prevO = Oprev_.as<K>();
+    }
+    q.keepD = keepD ? 1 : 0;
+    q.nu = par_.nu;
+    q.dt = dtCur_;
+    q.tiles = tiles_;
+    hipLaunchKernelGGL((dev::koAssemble<R>), dim3(tiles_.blocks), dim3(dev::kTileLanes), 0, stream_,
+                       koSystems(), q);
   }
 
   // BiCGStab iterations it0 .. it0 + k - 1 of n systems (passes of a system
@@ -2569,8 +2597,10 @@ class EngineT final : public Engine {
     const std::vector<int64_t> key = {4, curBuf_, preIbb_ ? 1 : 0, int64_t(options), B, kKoBatch};
     int rc = replay(key, [&] {
       for (int i = 0; i < kKoBatch; i++) {
+        // the fields that only the last step's values of are seen
+        const bool last = i == kKoBatch - 1;
         launchLB(options);
-        enqueueKoHead(true);
+        enqueueKoHead(last, last);
         enqueueIters(koSystems(), 2, 0, B, batchFlags_.as<int>() + 4 * i);
       }
     }, kKoBatch, err);

@@ -33,6 +33,7 @@ enum : uint32_t {
   kSolid = 0x0001,         // M_SOLID_NODE
   kIbbNode = 0x0002,       // node owns at least one interpolated link
   kSolidBoundary = 0x0004, // SOLID_BOUNDARY_NODE (k, omega pinned to 0)
+  kUnitDx = 0x0008,        // the four wall spacings are 1
   kPairUp = 0x0010,        // solver preconditioner: paired with the node above
   kPairDown = 0x0020,      // solver preconditioner: paired with the node below
   kBoundMask = 0xFF00,     // E_BOUND .. NW_BOUND, reference positions
@@ -1118,70 +1119,6 @@ struct KOParams {
   double nu, dt;
   TileMap tiles;
 };
-
-// Update_kOmega_Diffusivities (kOmegaKernels.cl:7-95).
-template <class M>
-__global__ __launch_bounds__(kBlockX) void koDiffusivities(
-    const uint16_t* __restrict__ mask, const double* __restrict__ K, const double* __restrict__ O,
-    const double* __restrict__ Nut, const double* __restrict__ Wd, double* __restrict__ Dk,
-    double* __restrict__ Do, double* __restrict__ F1a, double* __restrict__ dkdo,
-    const M* __restrict__ rho, const double* __restrict__ dX, KOParams p) {
-  using R = double;
-  int bx, y;
-  if (!tileOf(p.tiles, bx, y)) return;
-  const int x = bx * kBlockX + threadIdx.x;
-  if (x >= p.nX) return;
-  const size_t g = size_t(x) + size_t(p.XF) * y;
-  if (mask[g] & kSolid) return;
-  const size_t gw = x > 0 ? g - 1 : g + (p.nX - 1);
-  const size_t ge = x < p.nX - 1 ? g + 1 : g - x;
-  const size_t gn = g + p.XF, gs = g - p.XF;
-  const R in[ko::kDiffInputs] = {K[g],   K[ge],  K[gw],          K[gn],          K[gs],
-                                 O[g],   O[ge],  O[gw],          O[gn],          O[gs],
-                                 Nut[g], Wd[g],  R(rho[g]),      dX[g],          dX[g + p.D],
-                                 dX[g + 2 * p.D], dX[g + 3 * p.D]};
-  R o[ko::kDiffOutputs];
-  ko::koDiffT<R>(in, p.nu, o);
-  dkdo[g] = o[ko::kDiffMx];
-  dkdo[g + p.D] = o[ko::kDiffMy];
-  F1a[g] = o[ko::kDiffF1];
-  Dk[g] = o[ko::kDiffDk];
-  Do[g] = o[ko::kDiffDo];
-}
-
-// Update_kOmega_Coeffs_Implicit (kOmegaKernels.cl:187-480): normalised
-// five-point rows; A holds E, W, N, S planes (diagonal 1).
-struct KORows {
-  double Ak[4], Ao[4], bk, bo;
-};
-
-template <class M>
-__device__ __forceinline__ void koCoeffRow(
-    int x, size_t g, uint32_t m, const double* __restrict__ K, const double* __restrict__ O,
-    const double* __restrict__ Nut, const double* __restrict__ Dk, const double* __restrict__ Do,
-    const double* __restrict__ F1a, const double* __restrict__ dkdo, const double* __restrict__ Sx,
-    const M* __restrict__ rho, const M* __restrict__ uxa, const M* __restrict__ uya,
-    const double* __restrict__ dX, const double* __restrict__ Wd, const KOParams& p, KORows& o) {
-  using R = double;
-  const size_t gw = x > 0 ? g - 1 : g + (p.nX - 1);
-  const size_t ge = x < p.nX - 1 ? g + 1 : g - x;
-  const size_t gn = g + p.XF, gs = g - p.XF;
-  const R in[ko::kRowInputs] = {Dk[g],  Dk[ge],  Dk[gw],         Dk[gn],          Dk[gs],
-                                Do[g],  Do[ge],  Do[gw],         Do[gn],          Do[gs],
-                                dkdo[g], dkdo[g + p.D], R(uxa[g]), R(uya[g]),     R(rho[g]),
-                                K[g],   O[g],    F1a[g],         Nut[g],          Sx[g],
-                                Sx[g + p.D], Sx[g + 2 * p.D], Wd[g], dX[g],       dX[g + p.D],
-                                dX[g + 2 * p.D], dX[g + 3 * p.D]};
-  R out[ko::kRowOutputs];
-  ko::koRowT<R>(in, (m & kNesw) != 0, p.nu, p.dt, out);
-#pragma unroll
-  for (int d = 0; d < 4; d++) {
-    o.Ak[d] = out[ko::kRowAk + d];
-    o.Ao[d] = out[ko::kRowAo + d];
-  }
-  o.bk = out[ko::kRowBk];
-  o.bo = out[ko::kRowBo];
-}
 
 __device__ __forceinline__ void nbIndex(const KOParams& p, int x, size_t g, size_t (&nb)[4]) {
   nb[0] = x < p.nX - 1 ? g + 1 : g - x;        // E

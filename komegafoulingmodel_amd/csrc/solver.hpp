@@ -90,7 +90,7 @@ struct SolveSys {
   double* v[2];
   double* t;
   SolveState* st;   // [2]
-  double2* partial;  // [2][2 * nblk]
+  double2* partial;  // [2][2 * max(nblk, n0)]: sums by pass parity
   SolveState* out;  // the state the last finish kernel saw
   double rtol, atol;
   int maxit;
@@ -98,6 +98,7 @@ struct SolveSys {
   int nX, nY, XF;
   int64_t D;
   Strips s;
+  int n0;           // blocks of the assembly, whose sums open the solve
 };
 struct SolvePair {
   SolveSys sys[2];
@@ -184,11 +185,14 @@ __device__ __forceinline__ void blockSum2(Sum& a, Sum& b) {
 
 // A block's sums to (and all blocks' sums from) the partials of pass parity
 // `slot`: {a.hi, a.lo}, {b.hi, b.lo} per block.
+__device__ __forceinline__ double2* partialSlot(const SolveSys& y, int slot) {
+  return y.partial + size_t(slot) * 2 * max(y.s.nblk, y.n0);
+}
 template <int THREADS>
 __device__ __forceinline__ void writePartial(const SolveSys& y, int T, int slot, Sum a, Sum b) {
   blockSum2<THREADS>(a, b);
   if (threadIdx.x == 0) {
-    double2* out = y.partial + size_t(slot) * 2 * y.s.nblk + 2 * T;
+    double2* out = partialSlot(y, slot) + 2 * T;
     out[0] = make_double2(a.hi, a.lo);
     out[1] = make_double2(b.hi, b.lo);
   }
@@ -197,36 +201,24 @@ __device__ __forceinline__ void writePartial(const SolveSys& y, int T, int slot,
 // wave's loads return in order, and the sums must not wait behind the rows.
 template <int THREADS>
 struct Partials {
-  static constexpr int kAhead = 1;
-  double2 a[kAhead], b[kAhead];
-  __device__ __forceinline__ void load(const SolveSys& y, int slot) {
-    const double2* in = y.partial + size_t(slot) * 2 * y.s.nblk;
-#pragma unroll
-    for (int k = 0; k < kAhead; k++) {
-      const int i = int(threadIdx.x) + k * THREADS;
-      a[k] = b[k] = make_double2(0., 0.);
-      if (i < y.s.nblk) {
-        a[k] = in[2 * i];
-        b[k] = in[2 * i + 1];
-      }
+  double2 a, b;
+  __device__ __forceinline__ void load(const SolveSys& y, int slot, int n) {
+    const double2* in = partialSlot(y, slot);
+    const int i = int(threadIdx.x);
+    a = b = make_double2(0., 0.);
+    if (i < n) {
+      a = in[2 * i];
+      b = in[2 * i + 1];
     }
   }
-  __device__ __forceinline__ void sums(const SolveSys& y, int slot, double& outA, double& outB) const {
-    const double2* in = y.partial + size_t(slot) * 2 * y.s.nblk;
-    Sum p{}, q{};
-#pragma unroll
-    for (int k = 0; k < kAhead; k++) {
-      p.add(a[k].x);
-      p.lo += a[k].y;
-      q.add(b[k].x);
-      q.lo += b[k].y;
-    }
-    for (int i = int(threadIdx.x) + kAhead * THREADS; i < y.s.nblk; i += THREADS) {
+  __device__ __forceinline__ void sums(const SolveSys& y, int slot, int n, double& outA,
+                                       double& outB) const {
+    const double2* in = partialSlot(y, slot);
+    Sum p{a.x, a.y}, q{b.x, b.y};
+    for (int i = int(threadIdx.x) + THREADS; i < n; i += THREADS) {
       const double2 u = in[2 * i], v = in[2 * i + 1];
-      p.add(u.x);
-      p.lo += u.y;
-      q.add(v.x);
-      q.lo += v.y;
+      p.add(Sum{u.x, u.y});
+      q.add(Sum{v.x, v.y});
     }
     blockSum2<THREADS>(p, q);
     outA = p.value();
@@ -336,7 +328,7 @@ __device__ __forceinline__ bool beginPass(const SolveSys& y, const Partials<THRE
                                           int par, bool lead, SolveState& s) {
   __shared__ SolveState sh;
   double a, b;
-  in.sums(y, par, a, b);
+  in.sums(y, par, stage == 0 ? y.n0 : y.s.nblk, a, b);
   if (threadIdx.x == 0) {
     SolveState n{};
     if (stage != 0) n = y.st[par];
@@ -518,7 +510,7 @@ __global__ __launch_bounds__(kStripThreads) void solveApply(SolvePair P, int it,
   constexpr int stage = KIND == kPassFirstPV ? 0 : (KIND == kPassPV ? 3 : 1);
   if (passedOn(y, stage, par, c.T == 0)) return;
   Partials<kStripThreads> in;
-  in.load(y, par);
+  in.load(y, par, stage == 0 ? y.n0 : y.s.nblk);
   const ApplyPass<KIND> pass(y, c, it);
   typename ApplyPass<KIND>::Raw head, body;
   typename ApplyPass<KIND>::Coef co;
@@ -606,7 +598,7 @@ __global__ __launch_bounds__(kStripX) void solveUpdate(SolvePair P, int it, int 
   if (!chunkOf(y.s, y.nX, y.nY, c)) return;
   if (passedOn(y, 2, par, c.T == 0)) return;
   Partials<kStripX> in;
-  in.load(y, par);
+  in.load(y, par, y.s.nblk);
   const UpdatePass<FIRST> pass(y, c, it);
   typename UpdatePass<FIRST>::Raw q;
   const bool inner = int(threadIdx.x) < c.w;
@@ -630,8 +622,8 @@ __global__ __launch_bounds__(kStripX) void solveFinish(SolvePair P, int n, int p
     const SolveSys& y = P.sys[k];
     double a, b;
     Partials<kStripX> in;
-    in.load(y, par);
-    in.sums(y, par, a, b);
+    in.load(y, par, y.s.nblk);
+    in.sums(y, par, y.s.nblk, a, b);
     SolveState s = y.st[par];
     if (!s.done) advance(s, 3, a, b, y);
     if (threadIdx.x == 0) *y.out = s;
@@ -650,55 +642,242 @@ __global__ __launch_bounds__(kStripX) void solveFinish(SolvePair P, int n, int p
 // assembly: the rows and the first residual
 // ---------------------------------------------------------------------------
 
-// Calls f(x, y) for the nodes of this lane's column in the block's chunk.
-template <class F>
-__device__ __forceinline__ void forChunk(const Chunk& c, F&& f) {
-  if (int(threadIdx.x) >= c.w) return;
-  for (int k = c.y0; k < c.y1; k++) f(c.x0 + int(threadIdx.x), k);
+// The assembly kernels take tiles of 64 x 8 nodes with 256 lanes (two nodes
+// each), up to kTileBlocks blocks walking their XCD's run of tiles: the two per
+// CU that the k-omega assembly's registers allow, and few enough that the first
+// pass can add up their sums.
+constexpr int kTileX = 64, kTileY = 8, kTileLanes = 256, kTileBlocks = 512;
+constexpr int kTileStep = kTileLanes / kTileX;  // rows between a lane's two nodes
+struct Tiles {
+  int tilesX, nTiles, per, blocks;
+};
+inline Tiles tilesFor(int nX, int nY) {
+  Tiles t;
+  t.tilesX = (nX + kTileX - 1) / kTileX;
+  t.nTiles = t.tilesX * ((nY + kTileY - 1) / kTileY);
+  t.per = (t.nTiles + 7) / 8;
+  t.blocks = 8 * t.per < kTileBlocks ? 8 * t.per : kTileBlocks;
+  return t;
 }
 
-// Update_kOmega_Coeffs_Implicit (kOmegaKernels.cl:187-480): the normalised
-// rows of both systems, then the first residual r = b - A x from the current
-// K and O (the solve's initial guess); sums (r, r).  With prev set, K and O
-// are also kept there (the restart point of the step).
-template <class M>
-__global__ __launch_bounds__(kStripX) void koCoeffs(
-    const double* __restrict__ Nut, const double* __restrict__ Dk, const double* __restrict__ Do,
-    const double* __restrict__ F1a, const double* __restrict__ dkdo, const double* __restrict__ Sx,
-    const M* __restrict__ rho, const M* __restrict__ uxa, const M* __restrict__ uya,
-    const double* __restrict__ dX, const double* __restrict__ Wd, double* __restrict__ prevK,
-    double* __restrict__ prevO, SolvePair P, KOParams p) {
-  Chunk c;
-  if (!chunkOf(P.sys[0].s, p.nX, p.nY, c)) return;
-  Sum acc[2]{};
-  forChunk(c, [&](int x, int y) {
-    const size_t g = size_t(x) + size_t(p.XF) * y;
-    const uint32_t m = P.sys[0].mask[g];
-    if (m & kSolid) return;
-    KORows o;
-    koCoeffRow<M>(x, g, m, P.sys[0].x, P.sys[1].x, Nut, Dk, Do, F1a, dkdo, Sx, rho, uxa, uya, dX,
-                  Wd, p, o);
-    size_t nb[4];
-    nbIndex(p, x, g, nb);
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-      const double* A = v == 0 ? o.Ak : o.Ao;
-      const double* X = P.sys[v].x;
-      double* prev = v == 0 ? prevK : prevO;
-      if (prev) prev[g] = X[g];
-      double* Av = const_cast<double*>(P.sys[v].A);
-#pragma unroll
-      for (int d = 0; d < 4; d++) Av[g + size_t(d) * p.D] = A[d];
-      const double b = v == 0 ? o.bk : o.bo;
-      const double ax = X[g] + (A[0] * X[nb[0]] + A[1] * X[nb[1]] + A[2] * X[nb[2]] +
-                                A[3] * X[nb[3]]);
-      const double r = b - ax;
-      P.sys[v].r[0][g] = r;
-      acc[v].add(r * r);
-    }
+// Calls f(x0, y0) for the tiles of this block: the blocks of XCD k = blockIdx
+// % 8 walk the k-th run of tiles.
+template <class F>
+__device__ __forceinline__ void forTiles(const Tiles& t, F&& f) {
+  const int xcd = int(blockIdx.x & 7), stride = t.blocks >> 3;
+  const int end = min((xcd + 1) * t.per, t.nTiles);
+  for (int T = xcd * t.per + int(blockIdx.x >> 3); T < end; T += stride)
+    f((T % t.tilesX) * kTileX, (T / t.tilesX) * kTileY);
+}
+// Calls f(x, y) for this lane's nodes of every tile.
+template <class F>
+__device__ __forceinline__ void forTileNodes(const Tiles& t, int nX, int nY, F&& f) {
+  forTiles(t, [&](int x0, int y0) {
+    const int x = x0 + int(threadIdx.x) % kTileX, y = y0 + int(threadIdx.x) / kTileX;
+    if (x >= nX) return;
+    if (y < nY) f(x, y);
+    if (y + kTileStep < nY) f(x, y + kTileStep);
   });
-  writePartial<kStripX>(P.sys[0], c.T, 0, acc[0], Sum{});
-  writePartial<kStripX>(P.sys[1], c.T, 0, acc[1], Sum{});
+}
+
+// Difference weights of nodes whose four wall spacings are 1 (fdCoeffsT(1, 1)).
+#define KOFM_UNIT_WEIGHTS {0.5, -0.5, 0., 1., 1., -2.}
+
+// Marks the nodes whose four spacings are exactly 1: every fluid node that is
+// not next to a wall.  The assembly then neither reads the spacings (4 of its
+// planes) nor divides by them (24 divisions per node).
+__global__ __launch_bounds__(kBlockX) void unitSpacing(uint16_t* __restrict__ mask,
+                                                       const double* __restrict__ dX, int64_t D) {
+  const int64_t i = int64_t(blockIdx.x) * kBlockX + threadIdx.x;
+  if (i >= D) return;
+  const bool unit = dX[i] == 1. && dX[i + D] == 1. && dX[i + 2 * D] == 1. && dX[i + 3 * D] == 1.;
+  mask[i] = uint16_t((mask[i] & ~uint32_t(kUnitDx)) | (unit ? uint32_t(kUnitDx) : 0u));
+}
+
+// What the k-omega assembly reads and writes beside the systems.
+struct KOAssembly {
+  const double *nut, *S, *dX, *wd;
+  const void *rho, *ux, *uy;  // arithmetic type
+  double *Dk, *Do;            // diffusivities: read on solid nodes, written when keepD
+  double *F1, *dkdo;          // written when set (the adjoint's tape)
+  double *prevK, *prevO;      // when set, k and omega are kept there (restart point)
+  int keepD;
+  double nu, dt;
+  Tiles tiles;
+};
+
+// Update_kOmega_Diffusivities and Update_kOmega_Coeffs_Implicit
+// (kOmegaKernels.cl:7-95, 187-480): the diffusivities of a tile and the ring
+// around it go to LDS, then the normalised rows of both systems and the first
+// residual r = b - A x from the current k and omega (the solve's initial
+// guess); sums (r, r).  The ring's 144 evaluations beside the tile's 512 spare
+// the five diffusivity planes a write and a read.  A solid node keeps the
+// diffusivity it last had as a fluid node (zero if it never was).
+// Its registers leave two waves per SIMD, so a lane issues the loads of its
+// nodes together before it evaluates the first; then 4096 x 512 takes 106 us and
+// 2000 x 204 22 us, where separate diffusivity and row kernels took 166 and 30.
+// (Measured slower: a lane per node with extra waves for the ring, 116 and 36;
+// 16 x 16 tiles, 167 and 38; fewer registers by spilling, 206 and more.)
+template <class M>
+__global__ __launch_bounds__(kTileLanes) void koAssemble(SolvePair P, KOAssembly q) {
+  constexpr int RX = kTileX + 2, RY = kTileY + 2;
+  __shared__ double ldk[RX * RY], ldo[RX * RY];
+  const SolveSys& sy = P.sys[0];
+  const int nX = sy.nX, nY = sy.nY;
+  const int64_t XF = sy.XF, D = sy.D;
+  const uint16_t* __restrict__ mask = sy.mask;
+  const double* __restrict__ K = P.sys[0].x;
+  const double* __restrict__ O = P.sys[1].x;
+  const M* __restrict__ rho = static_cast<const M*>(q.rho);
+  const M* __restrict__ uxa = static_cast<const M*>(q.ux);
+  const M* __restrict__ uya = static_cast<const M*>(q.uy);
+  const double* __restrict__ dX = q.dX;
+  Sum acc[2]{};
+
+  // A node's diffusivity inputs; lanes without a node take node 0's values and
+  // use none, rows past the lattice the node's own.
+  struct Node {
+    size_t g;
+    uint32_t m;
+    double k[5], o[5], nut, wd, rho;
+  };
+  auto load = [&](Node& n, int x, int y, bool on) {
+    n.g = on ? size_t(x) + size_t(XF) * y : 0;
+    const size_t g = n.g;
+    const size_t nb[4] = {on ? (x < nX - 1 ? g + 1 : g - x) : g, on ? (x > 0 ? g - 1 : g + (nX - 1)) : g,
+                          on && y < nY - 1 ? g + XF : g, on && y > 0 ? g - XF : g};
+    n.m = mask[g];
+    if (!on) n.m = kSolid;
+    n.k[0] = K[g];
+    n.o[0] = O[g];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+      n.k[1 + d] = K[nb[d]];
+      n.o[1 + d] = O[nb[d]];
+    }
+    n.nut = q.nut[g];
+    n.wd = q.wd[g];
+    n.rho = double(rho[g]);
+  };
+  auto diff = [&](const Node& n, bool on, double (&d)[ko::kDiffOutputs]) {
+    if (n.m & kSolid) {
+      d[ko::kDiffDk] = on ? q.Dk[n.g] : 0.;
+      d[ko::kDiffDo] = on ? q.Do[n.g] : 0.;
+      return;
+    }
+    double in[ko::kDiffInputs] = {n.k[0], n.k[1], n.k[2], n.k[3], n.k[4], n.o[0],
+                                  n.o[1], n.o[2], n.o[3], n.o[4], n.nut,  n.wd,
+                                  n.rho,  1.,     1.,     1.,     1.};
+    if (n.m & kUnitDx) {
+      const double ax[6] = KOFM_UNIT_WEIGHTS, ay[6] = KOFM_UNIT_WEIGHTS;
+      ko::koDiffCore<double, double>(in, ax, ay, q.nu, d);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; c++) in[ko::kDiffDx + c] = dX[n.g + size_t(c) * D];
+      ko::koDiffT<double>(in, q.nu, d);
+    }
+  };
+
+  const int t = int(threadIdx.x);
+  const int ix = t % kTileX, iy = t / kTileX;
+  // this lane's ring node: the rows below and above, then the columns beside
+  // the tile (corners are not used); east of a tile that the lattice's edge
+  // cuts it follows the last column
+  const bool ring = t < 2 * kTileX + 2 * kTileY;
+  const int ringRow = t < 2 * kTileX ? (t < kTileX ? 0 : kTileY + 1) : 1 + t % kTileY;
+  const int ringCol = t < 2 * kTileX ? 1 + t % kTileX : (t < 2 * kTileX + kTileY ? 0 : -1);
+
+  forTiles(q.tiles, [&](int x0, int y0) {
+    const int w = min(kTileX, nX - x0);
+    Node n[2], e;
+    bool on[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int y = y0 + iy + kTileStep * i;
+      on[i] = ix < w && y < nY;
+      load(n[i], x0 + ix, y, on[i]);
+    }
+    const int ec = ringCol < 0 ? w + 1 : ringCol;
+    int ex = x0 + ec - 1;
+    ex = ex < 0 ? nX - 1 : (ex >= nX ? ex - nX : ex);
+    const int ey = y0 + ringRow - 1;
+    const bool eon = ring && (ec <= w || ringCol < 0) && ey >= 0 && ey < nY;
+    if (ring) load(e, ex, ey, eon);
+    double d[2][ko::kDiffOutputs];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      diff(n[i], on[i], d[i]);
+      const int c = (ix + 1) + RX * (iy + kTileStep * i + 1);
+      ldk[c] = d[i][ko::kDiffDk];
+      ldo[c] = d[i][ko::kDiffDo];
+      if (n[i].m & kSolid) continue;
+      if (q.keepD) {
+        q.Dk[n[i].g] = d[i][ko::kDiffDk];
+        q.Do[n[i].g] = d[i][ko::kDiffDo];
+      }
+      if (q.F1) {
+        q.F1[n[i].g] = d[i][ko::kDiffF1];
+        q.dkdo[n[i].g] = d[i][ko::kDiffMx];
+        q.dkdo[n[i].g + D] = d[i][ko::kDiffMy];
+      }
+    }
+    // (a cut tile's ring column may lie on a cell that an idle lane of the
+    // tile has just written)
+    if (w < kTileX) __syncthreads();
+    if (eon) {
+      double de[ko::kDiffOutputs];
+      diff(e, true, de);
+      ldk[ec + RX * ringRow] = de[ko::kDiffDk];
+      ldo[ec + RX * ringRow] = de[ko::kDiffDo];
+    }
+    double S[2][3], u[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) S[i][c] = q.S[n[i].g + size_t(c) * D];
+      u[i][0] = double(uxa[n[i].g]);
+      u[i][1] = double(uya[n[i].g]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      if (n[i].m & kSolid) continue;
+      const size_t g = n[i].g;
+      const int c = (ix + 1) + RX * (iy + kTileStep * i + 1);
+      double in[ko::kRowInputs] = {
+          d[i][ko::kDiffDk], ldk[c + 1], ldk[c - 1], ldk[c + RX], ldk[c - RX],
+          d[i][ko::kDiffDo], ldo[c + 1], ldo[c - 1], ldo[c + RX], ldo[c - RX],
+          d[i][ko::kDiffMx], d[i][ko::kDiffMy], u[i][0], u[i][1], n[i].rho, n[i].k[0], n[i].o[0],
+          d[i][ko::kDiffF1], n[i].nut, S[i][0], S[i][1], S[i][2], n[i].wd, 1., 1., 1., 1.};
+      double out[ko::kRowOutputs];
+      const bool nesw = (n[i].m & kNesw) != 0;
+      if (n[i].m & kUnitDx) {
+        const double ax[6] = KOFM_UNIT_WEIGHTS, ay[6] = KOFM_UNIT_WEIGHTS;
+        ko::koRowCore<double, double>(in, ax, ay, nesw, q.nu, q.dt, out);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) in[ko::kRowDx + j] = dX[g + size_t(j) * D];
+        ko::koRowT<double>(in, nesw, q.nu, q.dt, out);
+      }
+#pragma unroll
+      for (int v = 0; v < 2; v++) {
+        const double* A = out + (v == 0 ? ko::kRowAk : ko::kRowAo);
+        const double* X = v == 0 ? n[i].k : n[i].o;
+        double* prev = v == 0 ? q.prevK : q.prevO;
+        if (prev) prev[g] = X[0];
+        double* Av = const_cast<double*>(P.sys[v].A);
+#pragma unroll
+        for (int j = 0; j < 4; j++) Av[g + size_t(j) * D] = A[j];
+        const double ax = X[0] + (A[0] * X[1] + A[1] * X[2] + A[2] * X[3] + A[3] * X[4]);
+        const double r = out[v == 0 ? ko::kRowBk : ko::kRowBo] - ax;
+        P.sys[v].r[0][g] = r;
+        acc[v].add(r * r);
+      }
+    }
+    __syncthreads();
+  });
+  writePartial<kTileLanes>(P.sys[0], int(blockIdx.x), 0, acc[0], Sum{});
+  writePartial<kTileLanes>(P.sys[1], int(blockIdx.x), 0, acc[1], Sum{});
 }
 
 // ---------------------------------------------------------------------------
@@ -742,22 +921,25 @@ __device__ __forceinline__ void tWeights(double dp, double dm, bool testCentre, 
 // with T_in and the outlet column's E coefficient into the diagonal.  When
 // Tprev is set, T is also copied there (the restart point of the step).
 template <class M>
-__global__ __launch_bounds__(kStripX) void thermalCoeffs(
+__global__ __launch_bounds__(kTileLanes) void thermalCoeffs(
     const uint16_t* __restrict__ lbmask,
     const double* __restrict__ dX0, const double* __restrict__ Nut, const M* __restrict__ uxa,
     const M* __restrict__ uya, double* __restrict__ Tprev, SolvePair P, TParams tp, double dt,
-    KOParams p) {
+    KOParams p, Tiles tiles) {
   const SolveSys& sy = P.sys[0];
-  Chunk c;
-  if (!chunkOf(sy.s, p.nX, p.nY, c)) return;
   Sum rr{}, bb{};
-  forChunk(c, [&](int x, int y) {
+  forTileNodes(tiles, p.nX, p.nY, [&](int x, int y) {
     const size_t g = size_t(x) + size_t(p.XF) * y;
-    if (sy.mask[g] & kSolid) return;
+    const uint32_t m = sy.mask[g];
+    if (m & kSolid) return;
     const double* T = sy.x;
-    double dx1[3], dx2[3], dy1[3], dy2[3];
-    tWeights(dX0[g], dX0[g + p.D], true, dx1, dx2);
-    tWeights(dX0[g + 2 * p.D], dX0[g + 3 * p.D], false, dy1, dy2);
+    // spacings of 1: first differences (1/2, -1/2, 0), second (1, 1, -2)
+    double dx1[3] = {0.5, -0.5, 0.}, dx2[3] = {1., 1., -2.}, dy1[3] = {0.5, -0.5, 0.},
+           dy2[3] = {1., 1., -2.};
+    if (!(m & kUnitDx)) {
+      tWeights(dX0[g], dX0[g + p.D], true, dx1, dx2);
+      tWeights(dX0[g + 2 * p.D], dX0[g + 3 * p.D], false, dy1, dy2);
+    }
     size_t nb[4];
     nbIndex(p, x, g, nb);
     double alpha = (lbmask[g] & kSolid) ? tp.alphaFoul : tp.alphaFluid;
@@ -792,7 +974,7 @@ __global__ __launch_bounds__(kStripX) void thermalCoeffs(
     rr.add(r * r);
     bb.add(b * b);
   });
-  writePartial<kStripX>(sy, c.T, 0, rr, bb);
+  writePartial<kTileLanes>(sy, int(blockIdx.x), 0, rr, bb);
 }
 
 }  // namespace dev

@@ -1231,7 +1231,24 @@ class EngineT final : public Engine {
   // batches of k-omega steps (koBatch): the checkpoint of populations and
   // fields, the per-step done flags and iteration counts (device, pinned
   // host copy), and the steps still to run one at a time after a rollback
-  static constexpr int kKoBatch = 8, kKoSlack = 2, kKoBatchMaxIters = 16;
+  static constexpr int kKoBatch = 8, kKoBatchMaxIters = 16;
+  // Iterations each step of a batch is given: the most that a step of the
+  // last 128 needed; while that is above 4 (a start-up transient) the last
+  // solve's and two more, with the most of the last 16 kept.  A pass that finds
+  // its system done still costs its launch, 4.5 us in a chain (13.5 per spare
+  // iteration, of a 110 us step on 2000 x 204); one step in 128 that needs more
+  // costs a rollback of eight.
+  int predIters_ = 1, predWindow_ = 1, predAge_ = 0;
+  void noteIterations(int iters, int steps) {
+    predWindow_ = std::max(predWindow_, iters);
+    predIters_ = std::max(predIters_, predWindow_);
+    predAge_ += steps;
+    if (predAge_ < (predIters_ > 4 ? 16 : 128)) return;
+    predIters_ = predWindow_;
+    predWindow_ = std::max(1, iters);
+    predAge_ = 0;
+  }
+  int batchIters() const { return predIters_ > 4 ? std::max(1, lastIters_) + 2 : predIters_; }
   Buffer batchF_, batchKO_, batchM_, batchFlags_;
   int* hostFlags_ = nullptr;
   int koBatchHold_ = 0;
@@ -2543,8 +2560,8 @@ class EngineT final : public Engine {
   }
 
   // kKoBatch k-omega steps from one captured graph, the host polling once
-  // for all of them.  Each step gets the iterations the last solve needed
-  // plus kKoSlack (launches past convergence return at once) and records
+  // for all of them.  Each step gets the iterations that recent steps needed
+  // (batchIters; launches past convergence return at once) and records
   // whether its solves finished.  When every one did, the result is the
   // same as kKoBatch calls of koFullStep; otherwise (a solve needing more
   // iterations, a non-finite residual) the populations and fields go back
@@ -2553,7 +2570,7 @@ class EngineT final : public Engine {
   // step control.  Returns 1 when the batch ran, 0 when the caller should
   // step one at a time, or a negative error code.
   int koBatch(unsigned options, std::string& err) {
-    const int B = std::max(1, lastIters_) + kKoSlack;
+    const int B = batchIters();
     if (!useGraphs_ || stepsPerLB_ != 1 || injectNan_ || koBatchHold_ > 0 || B > kKoBatchMaxIters)
       return 0;
     const size_t D = size_t(D_);
@@ -2620,6 +2637,7 @@ class EngineT final : public Engine {
     }
     if (ok) {
       lastIters_ = iters;
+      noteIterations(iters, kKoBatch);
       prevValid_ = true;
       return 1;
     }
@@ -2753,6 +2771,7 @@ class EngineT final : public Engine {
     if (rc) return rc;
     nan = hostStatus_[0].nan || hostStatus_[1].nan;
     lastIters_ = std::max(hostStatus_[0].iters, hostStatus_[1].iters);
+    noteIterations(lastIters_, 1);
     return 0;
   }
 };

@@ -2486,6 +2486,11 @@ class EngineT final : public Engine {
   // diffusivity fields are written unless a later step of the same call
   // overwrites them, F1 and m grad k for the adjoint's tape only.
   void enqueueKoHead(bool savePrev = false, bool keepD = true, bool tape = false) {
+    hipLaunchKernelGGL((dev::koAssemble<R>), dim3(tiles_.blocks), dim3(dev::kTileLanes), 0, stream_,
+                       koSystems(), koAssembly(savePrev, keepD, tape));
+  }
+
+  dev::KOAssembly koAssembly(bool savePrev, bool keepD, bool tape) const {
     using K = double;
     dev::KOAssembly q{};
     q.nut = nut_.as<K>();
@@ -2509,8 +2514,7 @@ class EngineT final : public Engine {
     q.nu = par_.nu;
     q.dt = dtCur_;
     q.tiles = tiles_;
-    hipLaunchKernelGGL((dev::koAssemble<R>), dim3(tiles_.blocks), dim3(dev::kTileLanes), 0, stream_,
-                       koSystems(), q);
+    return q;
   }
 
   // BiCGStab iterations it0 .. it0 + k - 1 of n systems (passes of a system
@@ -2784,6 +2788,7 @@ class EnsembleT final : public Ensemble {
  public:
   explicit EnsembleT(std::vector<EngineT<S, R>*> m) : m_(std::move(m)) {
     ko_ = !m_.empty() && m_[0]->komega();
+    if (ko_) budget_ = 0;
     for (auto* e : m_) e->users_.push_back(this);
   }
   ~EnsembleT() override {
@@ -3033,9 +3038,11 @@ class EnsembleT final : public Ensemble {
     std::vector<int> builtParity;
     std::vector<uint64_t> builtGen;  // members' generations when the tables were built
 
-    // k-omega members: their solves' flags (pinned on the host), and the
-    // captured steps keyed by the iteration predictions and the entry parity
-    Buffer koFlags;
+    // k-omega members: the tables of their systems and assemblies, their
+    // solves' flags (pinned on the host), and the captured steps keyed by the
+    // iterations given and the entry parity
+    Buffer koSys, koAsm, koFlags;
+    unsigned koGridA = 0, koGridS = 0;  // blocks of the largest member
     int* koFlagsHost = nullptr;
     std::vector<std::pair<std::vector<int>, hipGraphExec_t>> koGraphs;
     int koShift = 0;
@@ -3160,6 +3167,26 @@ class EnsembleT final : public Ensemble {
       return 0;
     }
 
+    // the k-omega members' systems and assemblies
+    int fillSystems(std::string& err) {
+      std::vector<dev::SolvePair> sys;
+      std::vector<dev::KOAssembly> q;
+      koGridA = koGridS = 0;
+      for (auto* e : m) {
+        sys.push_back(e->koSystems());
+        q.push_back(e->koAssembly(false, true, false));
+        koGridA = std::max(koGridA, unsigned(e->tiles_.blocks));
+        koGridS = std::max(koGridS, unsigned(8 * e->strips_.per));
+      }
+      if (koSys.bytes() == 0) {
+        HIP_TRY(koSys.alloc(sys.size() * sizeof(sys[0])));
+        HIP_TRY(koAsm.alloc(q.size() * sizeof(q[0])));
+      }
+      HIP_TRY(hipMemcpy(koSys.as<void>(), sys.data(), sys.size() * sizeof(sys[0]), hipMemcpyHostToDevice));
+      HIP_TRY(hipMemcpy(koAsm.as<void>(), q.data(), q.size() * sizeof(q[0]), hipMemcpyHostToDevice));
+      return 0;
+    }
+
     void advance(int k) {
       for (auto* e : m) {
         if (k & 1) e->curBuf_ ^= 1;
@@ -3176,8 +3203,11 @@ class EnsembleT final : public Ensemble {
   int block_ = 512;
   int spp_ = 1;
   bool ko_ = false;  // every member runs k-omega
-  // population bytes (both buffers) per group; 0 puts every member in one
-  // launch.  The default fits the 256 MB last-level cache with room to spare.
+  // working-set bytes per group; 0 puts every member in one launch.  The
+  // default fits the 256 MB last-level cache with room to spare; k-omega
+  // members, whose step is a dozen launches for a group of any size, start as
+  // one group (six channels of 1.3 million nodes: 427 us a step, 678 in
+  // 160 MB groups).
   int64_t budget_ = int64_t(160) << 20;
 
   static int fail(std::string& err, const char* msg) {
@@ -3263,11 +3293,12 @@ class EnsembleT final : public Ensemble {
   }
 
   // ---- k-omega members ----
-  // Each step: one batched collide-stream launch over every member, then
-  // every member's k-omega solve (diffusivities, coefficients and as many
-  // iterations as its last solve needed), captured as one graph per entry
-  // parity and prediction; then one poll of every member's done flags, with
-  // chunks of four more iterations for the members not yet converged.
+  // Each step: one batched collide-stream launch over every member, one
+  // assembly launch and three launches per iteration over every member's
+  // systems (as many iterations as the last solves needed; systems that are
+  // done return at once), captured as one graph per entry parity and
+  // prediction; then one poll of every member's flags, with chunks of four
+  // more iterations while a member needs them.
   int stepKO(Group& g, int n, unsigned options, std::string& err) {
     const int nm = int(g.m.size());
     for (auto* e : g.m)
@@ -3293,21 +3324,44 @@ class EnsembleT final : public Ensemble {
         for (size_t i = 0; i < m.size(); i++) m[i]->stream_ = saved[i];
       }
     } swap(g.m, stream_);
-    auto solves = [&](const std::vector<int>& batch) {
-      for (int i = 0; i < nm; i++) {
-        g.m[i]->enqueueKoHead();
-        g.m[i]->enqueueIters(g.m[i]->koSystems(), 2, 0, batch[i],
-                             g.koFlags.template as<int>() + 4 * i);
+    // iterations it0 .. it0 + k - 1 of every member, then their flags
+    auto iterate = [&](int it0, int k) {
+      const auto* tab = g.koSys.template as<const dev::SolveSys>();
+      const dim3 grid(g.koGridS, unsigned(2 * nm)), blkA(dev::kStripThreads), blkU(dev::kStripX);
+      for (int it = it0; it < it0 + k; it++) {
+        const int par = (3 * it) & 1;
+        if (it == 0)
+          hipLaunchKernelGGL(dev::solveApplyTable<dev::kPassFirstPV>, grid, blkA, 0, stream_, tab, it, par);
+        else
+          hipLaunchKernelGGL(dev::solveApplyTable<dev::kPassPV>, grid, blkA, 0, stream_, tab, it, par);
+        hipLaunchKernelGGL(dev::solveApplyTable<dev::kPassST>, grid, blkA, 0, stream_, tab, it, par ^ 1);
+        if (it == 0)
+          hipLaunchKernelGGL(dev::solveUpdateTable<true>, grid, blkU, 0, stream_, tab, it, par);
+        else
+          hipLaunchKernelGGL(dev::solveUpdateTable<false>, grid, blkU, 0, stream_, tab, it, par);
       }
+      hipLaunchKernelGGL(dev::solveFinishTable, dim3(unsigned(nm)), blkU, 0, stream_, tab,
+                         (3 * (it0 + k)) & 1, g.koFlags.template as<int>());
     };
+    auto solves = [&](int batch) {
+      hipLaunchKernelGGL((dev::koAssembleTable<R>), dim3(g.koGridA, unsigned(nm)),
+                         dim3(dev::kTileLanes), 0, stream_,
+                         g.koSys.template as<const dev::SolvePair>(),
+                         g.koAsm.template as<const dev::KOAssembly>());
+      iterate(0, batch);
+    };
+    int maxIt = 1;
+    for (auto* e : g.m) maxIt = std::max({maxIt, e->par_.maxIters[0], e->par_.maxIters[1]});
     for (int s = 0; s < n; s++) {
-      std::vector<int> batch(nm);
-      for (int i = 0; i < nm; i++) batch[i] = std::min(std::max(1, g.m[i]->lastIters_), 8);
+      // every member is given the most that one's last solve needed
+      int batch = 1;
+      for (auto* e : g.m) batch = std::max(batch, std::min(e->lastIters_, 8));
       bool fresh = false;
       for (auto* e : g.m) fresh |= !e->preIbb_;
       if (fresh) {
         // the first step after an upload, without the pending correction
         int rc = g.fill(*this, g.eager, options, 0, true, false, g.eagerTiles, err);
+        if (!rc) rc = g.fillSystems(err);
         if (rc) return rc;
         launch(g.eager, g.eagerTiles, nm, false);
         solves(batch);
@@ -3321,6 +3375,7 @@ class EnsembleT final : public Ensemble {
             g.builtGen != g.gens()) {
           int rc = g.fill(*this, g.ents[0], options, 0, false, false, g.totalTiles, err);
           if (!rc) rc = g.fill(*this, g.ents[1], options, 1, false, false, g.totalTiles, err);
+          if (!rc) rc = g.fillSystems(err);
           if (rc) return rc;
           g.dropKOGraphs();
           g.built = true;
@@ -3329,8 +3384,7 @@ class EnsembleT final : public Ensemble {
           g.builtGen = g.gens();
           g.koShift = 0;
         }
-        std::vector<int> key(batch);
-        key.push_back(g.koShift & 1);
+        const std::vector<int> key = {batch, g.koShift & 1};
         hipGraphExec_t exec = nullptr;
         for (auto& c : g.koGraphs)
           if (c.first == key) exec = c.second;
@@ -3348,8 +3402,8 @@ class EnsembleT final : public Ensemble {
         HIP_TRY(hipGraphLaunch(exec, stream_));
         g.koShift++;
       }
-      // poll every member; more iterations where needed
-      std::vector<int> it(batch);
+      // poll every member; more iterations while one needs them
+      int it = batch;
       const int* flags = g.koFlagsHost;
       while (true) {
         HIP_TRY(hipMemcpyAsync(g.koFlagsHost, g.koFlags.template as<void>(), 4 * size_t(nm) * sizeof(int),
@@ -3361,17 +3415,12 @@ class EnsembleT final : public Ensemble {
             err = "non-finite residual in the k-omega solve of an ensemble member";
             return KOFM_ERR_SOLVER_NAN;
           }
-          const EngineT<S, R>* e = g.m[i];
-          const int maxIt = std::max(e->par_.maxIters[0], e->par_.maxIters[1]);
-          if (!flags[4 * i] && it[i] < maxIt) {
-            const int k = std::min(4, maxIt - it[i]);
-            g.m[i]->enqueueIters(g.m[i]->koSystems(), 2, it[i], k,
-                                 g.koFlags.template as<int>() + 4 * i);
-            it[i] += k;
-            more = true;
-          }
+          more = more || !flags[4 * i];
         }
-        if (!more) break;
+        if (!more || it >= maxIt) break;
+        const int k = std::min(4, maxIt - it);
+        iterate(it, k);
+        it += k;
       }
       for (int i = 0; i < nm; i++) g.m[i]->lastIters_ = flags[4 * i + 2];
       for (auto* e : g.m) {

@@ -500,11 +500,8 @@ struct ApplyPass {
   }
 };
 
-// The passes: grid.x covers the chunks (8 * per blocks), grid.y the systems.
-// it: the iteration, par: the pass parity.
 template <int KIND>
-__global__ __launch_bounds__(kStripThreads) void solveApply(SolvePair P, int it, int par) {
-  const SolveSys& y = P.sys[blockIdx.y];
+__device__ __forceinline__ void applyBlock(const SolveSys& y, int it, int par) {
   Chunk c;
   if (!chunkOf(y.s, y.nX, y.nY, c)) return;
   constexpr int stage = KIND == kPassFirstPV ? 0 : (KIND == kPassPV ? 3 : 1);
@@ -522,6 +519,19 @@ __global__ __launch_bounds__(kStripThreads) void solveApply(SolvePair P, int it,
   Sum a{}, b{};
   pass.run(s, head, body, co, a, b);
   writePartial<kStripThreads>(y, c.T, par ^ 1, a, b);
+}
+
+// The passes: grid.x covers the chunks (8 * per blocks), grid.y the systems,
+// which are the launch's arguments or, for the members of an ensemble, a table
+// (grid.x then covers the largest).  it: the iteration, par: the pass parity.
+template <int KIND>
+__global__ __launch_bounds__(kStripThreads) void solveApply(SolvePair P, int it, int par) {
+  applyBlock<KIND>(P.sys[blockIdx.y], it, par);
+}
+template <int KIND>
+__global__ __launch_bounds__(kStripThreads) void solveApplyTable(const SolveSys* __restrict__ tab,
+                                                                 int it, int par) {
+  applyBlock<KIND>(tab[blockIdx.y], it, par);
 }
 
 // XR over one chunk, four rows at a time so that their loads overlap.
@@ -592,8 +602,7 @@ struct UpdatePass {
 };
 
 template <bool FIRST>
-__global__ __launch_bounds__(kStripX) void solveUpdate(SolvePair P, int it, int par) {
-  const SolveSys& y = P.sys[blockIdx.y];
+__device__ __forceinline__ void updateBlock(const SolveSys& y, int it, int par) {
   Chunk c;
   if (!chunkOf(y.s, y.nX, y.nY, c)) return;
   if (passedOn(y, 2, par, c.T == 0)) return;
@@ -609,17 +618,26 @@ __global__ __launch_bounds__(kStripX) void solveUpdate(SolvePair P, int it, int 
   if (inner) pass.run(s, q, a, b);
   writePartial<kStripX>(y, c.T, par ^ 1, a, b);
 }
+template <bool FIRST>
+__global__ __launch_bounds__(kStripX) void solveUpdate(SolvePair P, int it, int par) {
+  updateBlock<FIRST>(P.sys[blockIdx.y], it, par);
+}
+template <bool FIRST>
+__global__ __launch_bounds__(kStripX) void solveUpdateTable(const SolveSys* __restrict__ tab, int it,
+                                                            int par) {
+  updateBlock<FIRST>(tab[blockIdx.y], it, par);
+}
 
 // After the last XR launched (parity par): takes its sums in and leaves every
 // system's state in `out`; with flags, flags[0] = 1 when all have finished,
 // flags[1] = 1 when one met a non-finite residual, flags[2] = the iterations
 // they took.  The pass state is left alone, so more iterations may follow.
-// One block.
-__global__ __launch_bounds__(kStripX) void solveFinish(SolvePair P, int n, int par,
-                                                       int* __restrict__ flags) {
+// One block per lattice.
+__device__ __forceinline__ void finishBlock(const SolveSys* __restrict__ sys, int n, int par,
+                                            int* __restrict__ flags) {
   int done = 1, nan = 0, iters = 0;
   for (int k = 0; k < n; k++) {
-    const SolveSys& y = P.sys[k];
+    const SolveSys& y = sys[k];
     double a, b;
     Partials<kStripX> in;
     in.load(y, par, y.s.nblk);
@@ -636,6 +654,15 @@ __global__ __launch_bounds__(kStripX) void solveFinish(SolvePair P, int n, int p
     flags[1] = nan;
     flags[2] = iters;
   }
+}
+__global__ __launch_bounds__(kStripX) void solveFinish(SolvePair P, int n, int par,
+                                                       int* __restrict__ flags) {
+  finishBlock(P.sys, n, par, flags);
+}
+// two systems and four flags per member
+__global__ __launch_bounds__(kStripX) void solveFinishTable(const SolveSys* __restrict__ tab, int par,
+                                                            int* __restrict__ flags) {
+  finishBlock(tab + 2 * blockIdx.x, 2, par, flags + 4 * blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -719,7 +746,8 @@ struct KOAssembly {
 // (Measured slower: a lane per node with extra waves for the ring, 116 and 36;
 // 16 x 16 tiles, 167 and 38; fewer registers by spilling, 206 and more.)
 template <class M>
-__global__ __launch_bounds__(kTileLanes) void koAssemble(SolvePair P, KOAssembly q) {
+__device__ __forceinline__ void assembleBlock(const SolvePair& P, const KOAssembly& q) {
+  if (int(blockIdx.x) >= q.tiles.blocks) return;
   constexpr int RX = kTileX + 2, RY = kTileY + 2;
   __shared__ double ldk[RX * RY], ldo[RX * RY];
   const SolveSys& sy = P.sys[0];
@@ -878,6 +906,16 @@ __global__ __launch_bounds__(kTileLanes) void koAssemble(SolvePair P, KOAssembly
   });
   writePartial<kTileLanes>(P.sys[0], int(blockIdx.x), 0, acc[0], Sum{});
   writePartial<kTileLanes>(P.sys[1], int(blockIdx.x), 0, acc[1], Sum{});
+}
+template <class M>
+__global__ __launch_bounds__(kTileLanes) void koAssemble(SolvePair P, KOAssembly q) {
+  assembleBlock<M>(P, q);
+}
+// member blockIdx.y of an ensemble
+template <class M>
+__global__ __launch_bounds__(kTileLanes) void koAssembleTable(const SolvePair* __restrict__ P,
+                                                              const KOAssembly* __restrict__ q) {
+  assembleBlock<M>(P[blockIdx.y], q[blockIdx.y]);
 }
 
 // ---------------------------------------------------------------------------

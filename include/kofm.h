@@ -532,7 +532,8 @@ int kofm_save_debug(kofm_ctx* ctx, const char* dir);
  * neighbouring nodes per lane; the tile width must divide nX) and the
  * padding (elements,
  * multiple of 64) between the nine population planes in HBM.  The state is preserved and
- * every shape gives bit-identical results.  No counterpart in the reference,
+ * every shape gives bit-identical results.  Until a shape is set, plain steps
+ * take two steps per pass where that is the faster for the lattice's size.  No counterpart in the reference,
  * whose work-group is fixed at 128 x 1 (ConstDef.h:70-79). */
 int kofm_set_launch(kofm_ctx* ctx, int32_t block_x, int32_t nodes_per_lane,
                     int32_t steps_per_pass, int64_t plane_pad);

@@ -670,7 +670,7 @@ class EngineT final : public Engine {
       }
     }
     while (s < n) {
-      if (!ko_ && lbSpp_ == 2 && n - s >= 2) {
+      if (!ko_ && stepsPerPass() == 2 && n - s >= 2) {
         launchLB2(options);
         s += 2;
         continue;
@@ -741,7 +741,7 @@ class EngineT final : public Engine {
     for (int s = 0; s < n; launches++) {
       HIP_TRY(hipEventRecord(evs_[2 + 2 * launches], stream_));
       int rc = 0;
-      if (!ko_ && lbSpp_ == 2 && n - s >= 2) {
+      if (!ko_ && stepsPerPass() == 2 && n - s >= 2) {
         launchLB2(options);
         s += 2;
       } else {
@@ -1303,6 +1303,7 @@ class EngineT final : public Engine {
   int lbBlock_ = 512;   // work-group width of the collide-stream kernel
   int lbNpt_ = 1;       // lattice nodes per lane (1, or 2 neighbouring nodes)
   int lbSpp_ = 1;       // plain steps per pass (2: the temporally blocked kernel)
+  bool autoLaunch_ = true;  // no shape was set: plain steps take autoTile()
   bool ko_;
   hipStream_t stream_ = nullptr;
   Buffer fA_, fB_, mask_, ibbIdx_, ibbQ_, rho_, ux_, uy_;
@@ -1737,7 +1738,7 @@ class EngineT final : public Engine {
     const int buf0 = curBuf_;
     hipGraph_t graph = nullptr;
     HIP_TRY(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    if (lbSpp_ == 2)
+    if (stepsPerPass() == 2)
       for (int k = 0; k < kGraphSteps / 2; k++) launchLB2(options);
     else
       for (int k = 0; k < kGraphSteps; k++) launchLB(options);
@@ -1757,7 +1758,7 @@ class EngineT final : public Engine {
   void forwardSegment(int len, int w0, const dev::ObjectiveNodes& on) {
     const dim3 og((on.n + 63) / 64);
     int m = 0;
-    if (lbSpp_ == 2)  // steps before the window need no objective term
+    if (stepsPerPass() == 2)  // steps before the window need no objective term
       for (; m + 2 <= w0; m += 2) launchLB2(0);
     for (; m < len; m++) {
       const S* src = cur();
@@ -1778,7 +1779,7 @@ class EngineT final : public Engine {
     // recompute every state of the segment; with a two-step launch shape the
     // pairs run the temporally blocked kernel that also writes the middle state
     int m = 0;
-    if (lbSpp_ == 2 && lbNpt_ == 1 && nX_ % 64 == 0) {
+    if (stepsPerPass() == 2 && lbNpt_ == 1) {
       for (; m + 2 <= len; m += 2) {
         auto pA = lbParams(0);
         pA.applyIbb = m == 0 ? ap0 : 1;
@@ -2149,7 +2150,7 @@ class EngineT final : public Engine {
     auto p = lbParams(0);
     p.applyIbb = apply;
     p.saveMacros = 0;
-    launchLBBlock<false>(lbBlock_, lbNpt_, p, src, dst);
+    launchLBBlock<false>(autoLaunch_ ? 256 : lbBlock_, lbNpt_, p, src, dst);
   }
 
   // The temporally blocked kernels, selected by the tile's node count: one
@@ -2182,7 +2183,7 @@ class EngineT final : public Engine {
   void launchT2T(const dev::LBParams<R>& pA, const dev::LBParams<R>& pB, const S* src, S* dst,
                  S* mid1 = nullptr) {
     dev::TileMap tm;
-    tm.tilesX = nX_ / TX;
+    tm.tilesX = (nX_ + TX - 1) / TX;
     tm.nTiles = tm.tilesX * ((nY_ + TY - 1) / TY);
     tm.per = (tm.nTiles + 7) / 8;
     hipLaunchKernelGGL((dev::lbCollideStreamT2<S, R, TX, TY>), dim3(8 * tm.per),
@@ -2211,6 +2212,27 @@ class EngineT final : public Engine {
     }
   }
 
+  // The two-step tile of plain steps when no launch shape was set, by the
+  // lattice's size (0: one step per pass).  Every shape gives the same bits.
+  // Measured per step, one step per pass of 512 lanes against this tile, FP32
+  // (FP64): 257 x 61 4.1 -> 3.1 us (4.3 -> 3.3) with 64 x 8, 2001 x 203 10.7 ->
+  // 5.7 (13.5 -> 8.8) with 64 x 13, 1500 x 467 12.7 -> 9.2 (18.7 -> 13.4) and 3001 x
+  // 600 26.3 -> 18.5 (47.9 -> 30.1) with 64 x 29, 8192 x 1024 FP32 119 -> 76 with
+  // the node pairs of 128 x 12 (94 with 64 x 29).  FP16: 1984 x 203 7.9 -> 4.7 and
+  // 1472 x 467 11.1 -> 7.9 with 64 x 13, 2048 x 600 13.2 -> 10.0 with the node pairs
+  // of 64 x 26 (12.0 with 64 x 13); a large odd width is no faster in two-step
+  // tiles (4096 x 512: 17.7, 18.6 to 21.8).  A small lattice needs many blocks, a
+  // large one little ring.
+  int autoTile() const {
+    if (ko_ || kSR) return 0;
+    const int64_t n = int64_t(nX_) * nY_;
+    if (n < 50000) return 512;
+    if (sizeof(S) == 2) return n < 1000000 ? 832 : (nX_ % 64 == 0 ? 1664 : 0);
+    if (n < 600000) return 832;
+    return sizeof(S) == 4 && nX_ % 128 == 0 && n >= 4000000 ? 1536 : 1856;
+  }
+  int stepsPerPass() const { return autoLaunch_ ? (autoTile() ? 2 : 1) : lbSpp_; }
+
   // Two plain steps in one pass (k-omega off); the macros, if asked for,
   // are the second step's.
   void launchLB2(unsigned options) {
@@ -2219,7 +2241,7 @@ class EngineT final : public Engine {
     auto pB = lbParams(options);
     pB.applyIbb = 1;
     pB.seed = pA.seed + 1;
-    launchT2(lbBlock_, pA, pB, cur(), other());
+    launchT2(autoLaunch_ ? autoTile() : lbBlock_, pA, pB, cur(), other());
     curBuf_ ^= 1;
     preIbb_ = true;
     stepCount_ += 2;
@@ -2230,7 +2252,7 @@ class EngineT final : public Engine {
     if (ko_)
       launchLBBlock<true>(lbBlock_, lbNpt_, p, cur(), other());
     else
-      launchLBBlock<false>(lbBlock_, lbNpt_, p, cur(), other());
+      launchLBBlock<false>(autoLaunch_ ? 256 : lbBlock_, lbNpt_, p, cur(), other());
     curBuf_ ^= 1;
     preIbb_ = true;
     stepCount_++;
@@ -2290,6 +2312,7 @@ class EngineT final : public Engine {
     if (pad < 0 || pad % 64) return fail(err, "plane padding must be a non-negative multiple of 64");
     int rc = relayout(pad, err);
     if (rc) return rc;
+    autoLaunch_ = false;
     lbBlock_ = block;
     lbNpt_ = npt;
     lbSpp_ = spp;
@@ -2315,6 +2338,7 @@ class EngineT final : public Engine {
     bestSpp = lbSpp_;
     bestPad = P_ - D_;
     int rc = 0;
+    bool bestOwn = false;
     for (int64_t pad : pads) {
       if (!popsFit(D_ + pad)) continue;
       Buffer a, b;
@@ -2345,11 +2369,15 @@ class EngineT final : public Engine {
             bestNpt = npt;
             bestSpp = 1;
             bestPad = pad;
+            bestOwn = false;
           }
         }
       if (!ko_ && !kSR)
         for (int block : {512, 640, 832, 1856, 1024, 1536, 1664, 3584}) {
-          if (!t2Tile(block) || nX_ % t2Width(block)) continue;
+          // of widths that are no multiple of a tile's, the size's own tile (the
+          // launch without a set shape) is a candidate
+          const bool own = nX_ % 64 && block == autoTile();
+          if (!own && (!t2Tile(block) || nX_ % t2Width(block))) continue;
           auto pA = p, pB = p;
           pA.applyIbb = 1;
           launchT2(block, pA, pB, a.as<S>(), b.as<S>());  // warm-up
@@ -2368,6 +2396,7 @@ class EngineT final : public Engine {
             bestNpt = 1;
             bestSpp = 2;
             bestPad = pad;
+            bestOwn = own;
           }
         }
     }
@@ -2375,7 +2404,14 @@ class EngineT final : public Engine {
     (void)hipEventDestroy(e1);
     HIP_TRY(hipGetLastError());
     if (rc) return rc;
-    return setLaunch(bestBlock, bestNpt, bestSpp, bestPad, err);
+    if (!bestOwn) return setLaunch(bestBlock, bestNpt, bestSpp, bestPad, err);
+    // the launch without a set shape, reported as the one-step shape that
+    // kofm_set_launch takes on such a width
+    bestBlock = 256;
+    bestSpp = 1;
+    rc = setLaunch(bestBlock, 1, 1, bestPad, err);
+    if (!rc) autoLaunch_ = true;
+    return rc;
   }
 
  private:

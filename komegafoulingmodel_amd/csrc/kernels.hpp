@@ -573,7 +573,8 @@ __device__ __forceinline__ bool tileOf(const TileMap& t, int& bx, int& by) {
 // two steps per pass (temporal blocking)
 // ---------------------------------------------------------------------------
 
-// Two plain steps in one pass over a TX x TY tile (nX % TX == 0).  The first
+// Two plain steps in one pass over a TX x TY tile (the last tile of a row may
+// be cut by the lattice's edge: its ring column east is then column 0).  The first
 // step runs on the tile plus a one-node ring, reading the stored
 // populations from HBM and pushing into LDS; the second runs on the tile,
 // reading LDS and pushing to HBM.  The intermediate populations never touch
@@ -611,10 +612,11 @@ __device__ __forceinline__ void t2Tile(const S* __restrict__ src, S* __restrict_
   const KOFields none{nullptr, nullptr, nullptr, nullptr, nullptr};
 
   // step 1 on the tile and its ring
+  const int w = min(TX, pA.nX - x0);  // the tile's own columns
   for (int r = threadIdx.x; r < NR; r += t2Lanes<TX, TY>()) {
     const int rx = r % RX, ry = r / RX;
     const int y = y0 - 1 + ry;
-    if (y < 0 || y >= pA.nY) continue;
+    if (y < 0 || y >= pA.nY || rx > w + 1) continue;
     int x = x0 - 1 + rx;
     x = x < 0 ? x + pA.nX : (x >= pA.nX ? x - pA.nX : x);
     const size_t gi = size_t(x) + size_t(pA.XF) * y;
@@ -623,7 +625,7 @@ __device__ __forceinline__ void t2Tile(const S* __restrict__ src, S* __restrict_
     R g[9];
     loadNode<S, R>(g, src, gi, x, y, m, ibbIdx, ibbQ, pA);
     collideNode<R, false, kWideMoments<S, R>>(g, gi, rhoOut, uxOut, uyOut, none, pA);
-    if (mid1 && rx >= 1 && rx <= TX && ry >= 1 && ry <= TY) {
+    if (mid1 && rx >= 1 && rx <= w && ry >= 1 && ry <= TY) {
       const int xe = x < pA.nX - 1 ? x + 1 : 0;
       const int xw = x > 0 ? x - 1 : pA.nX - 1;
 #pragma unroll
@@ -662,7 +664,7 @@ __device__ __forceinline__ void t2Tile(const S* __restrict__ src, S* __restrict_
   for (int q = threadIdx.x; q < TX * TY; q += t2Lanes<TX, TY>()) {
     const int ix = q % TX, iy = q / TX;
     const int x = x0 + ix, y = y0 + iy;
-    if (y >= pB.nY) continue;
+    if (y >= pB.nY || ix >= w) continue;
     const size_t gi = size_t(x) + size_t(pB.XF) * y;
     const uint32_t m = mask[gi];
     if (m & kSolid) continue;

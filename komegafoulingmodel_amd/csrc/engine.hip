@@ -771,16 +771,13 @@ class EngineT final : public Engine {
     if (!haveState_) return fail(err, "state not initialised");
     const int nSS = int(geo_.ss.size()), nb = geo_.nBLshear();
     auto p = lbParams(0);
-    if (nSS > 0) {
-      hipLaunchKernelGGL((dev::shearNodes<S, R>), dim3((nSS + 63) / 64), dim3(64), 0, stream_,
-                         cur(), mask_.as<uint16_t>(), ibbIdx_.as<int32_t>(), ibbQ_.as<R>(),
+    const int nodeBlocks = (nSS + 63) / 64, linkBlocks = (4 * nb + 63) / 64;
+    if (nodeBlocks + linkBlocks > 0) {
+      hipLaunchKernelGGL((dev::wallShear<S, R>), dim3(unsigned(nodeBlocks + linkBlocks)), dim3(64), 0,
+                         stream_, cur(), mask_.as<uint16_t>(), ibbIdx_.as<int32_t>(), ibbQ_.as<R>(),
                          ss_.as<int32_t>(), nSS, cfss_.as<R>(), rho_.as<R>(), ux_.as<R>(),
-                         uy_.as<R>(), ko_ ? (const double*)nut_.as<double>() : nullptr, tau_.as<R>(), p);
-      HIP_TRY(hipGetLastError());
-    }
-    if (nb > 0) {
-      hipLaunchKernelGGL((dev::shearLinks<R>), dim3((nb + 63) / 64), dim3(64), 0, stream_,
-                         wts_.as<R>(), sInd_.as<int32_t>(), tau_.as<R>(), nb, tauBL_.as<R>());
+                         uy_.as<R>(), ko_ ? (const double*)nut_.as<double>() : nullptr, tau_.as<R>(),
+                         wts_.as<R>(), sInd_.as<int32_t>(), nb, tauBL_.as<R>(), nodeBlocks, p);
       HIP_TRY(hipGetLastError());
     }
     return 0;

@@ -1129,7 +1129,7 @@ __device__ __forceinline__ void nbIndex(const KOParams& p, int x, size_t g, size
   nb[3] = g - p.XF;                            // S
 }
 
-// K, O of every non-solid node back from the copies koCoeffs kept at the
+// K, O of every non-solid node back from the copies koAssemble kept at the
 // start of the step (kOmega::halveTimeStep's copyFromPrevSolution,
 // kOmega.cpp:387-399, GMRESSolver.cpp:1470-1476).
 __global__ __launch_bounds__(kBlockX) void koRestore(const uint16_t* __restrict__ mask,
@@ -1202,41 +1202,45 @@ __device__ __forceinline__ R wallTraction(const R (&g)[9], R r, R ux, R uy,
   return tx < R(0) ? -t : t;
 }
 
-// TR_shear_1 (trKernelsShear.cl:174-222): traction at wall nodes from the
-// newest populations (with the pending interpolated bounce-back) and the
-// stored macros.
+// TR_shear_1 and TR_shear_2 (trKernelsShear.cl:174-222, 300-316): traction at
+// wall nodes from the newest populations (with the pending interpolated
+// bounce-back) and the stored macros, and the boundary links' shear from the
+// tractions of their four nodes.  One launch: its first nodeBlocks blocks take
+// a node per lane; in the others four lanes evaluate the four nodes of a link
+// again, because a second launch that waits for the tractions costs 4.7 us and
+// the nodes (a few thousand, in L2) next to nothing: 100 calls after three steps
+// each on 2001 x 203 took 5.50 ms in all with two launches, 5.29 with one.
 template <class S, class R>
-__global__ __launch_bounds__(64) void shearNodes(
+__global__ __launch_bounds__(64) void wallShear(
     const S* __restrict__ src, const uint16_t* __restrict__ mask,
     const int32_t* __restrict__ ibbIdx, const R* __restrict__ ibbQ,
     const int32_t* __restrict__ ss, int nSS, const R* __restrict__ cfss,
     const R* __restrict__ rho, const R* __restrict__ uxa, const R* __restrict__ uya,
-    const double* __restrict__ nut, R* __restrict__ tau, LBParams<R> p) {
-  const int n = blockIdx.x * 64 + threadIdx.x;
-  if (n >= nSS) return;
-  const int gi = ss[n];
-  const int x = gi % p.XF, y = gi / p.XF;
-  R g[9];
-  loadNode<S, R>(g, src, size_t(gi), x, y, mask[gi], ibbIdx, ibbQ, p);
-  tau[n] = wallTraction<R>(g, rho[gi], uxa[gi], uya[gi], cfss + 16 * size_t(n),
+    const double* __restrict__ nut, R* __restrict__ tau, const R* __restrict__ w,
+    const int32_t* __restrict__ sInd, int nb, R* __restrict__ blTau, int nodeBlocks, LBParams<R> p) {
+  auto traction = [&](int n) {
+    const int gi = ss[n];
+    const int x = gi % p.XF, y = gi / p.XF;
+    R g[9];
+    loadNode<S, R>(g, src, size_t(gi), x, y, mask[gi], ibbIdx, ibbQ, p);
+    return wallTraction<R>(g, rho[gi], uxa[gi], uya[gi], cfss + 16 * size_t(n),
                            shearScale<R>(nut ? R(nut[gi]) : R(0), p.nu));
-}
-
-// TR_shear_2 (trKernelsShear.cl:300-316).
-template <class R>
-__global__ __launch_bounds__(64) void shearLinks(const R* __restrict__ w,
-                                                 const int32_t* __restrict__ sInd,
-                                                 const R* __restrict__ tau, int nb,
-                                                 R* __restrict__ blTau) {
-  const int n = blockIdx.x * 64 + threadIdx.x;
-  if (n >= nb) return;
+  };
+  if (int(blockIdx.x) < nodeBlocks) {
+    const int n = blockIdx.x * 64 + threadIdx.x;
+    if (n < nSS) tau[n] = traction(n);
+    return;
+  }
+  const int e = (int(blockIdx.x) - nodeBlocks) * 64 + int(threadIdx.x);  // 4 link + slot
+  const bool on = e < 4 * nb;
+  const int i = on ? sInd[e] : -1;
+  const R v = on ? w[e] * (i >= 0 ? traction(i) : R(0)) : R(0);
+  // the link's sum in slot order, in its first lane
+  const int first = int(threadIdx.x) & ~3;
   R s = R(0);
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int i = sInd[4 * n + k];
-    s += w[4 * n + k] * (i >= 0 ? tau[i] : R(0));
-  }
-  blTau[n] = s;
+  for (int k = 0; k < 4; k++) s += __shfl(v, first + k, 64);
+  if (on && (e & 3) == 0) blTau[e >> 2] = s;
 }
 
 // ---------------------------------------------------------------------------

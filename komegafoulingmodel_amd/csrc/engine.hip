@@ -12,16 +12,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <initializer_list>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "../../include/kofm.h"
 #include "engine.hpp"
+#include "fetch.hpp"
 #include "adjoint.hpp"
 #include "kernels.hpp"
 #include "nusselt.hpp"
@@ -73,103 +71,6 @@ class Buffer {
  private:
   void* p_ = nullptr;
   size_t bytes_ = 0;
-};
-
-// Pinned host memory that fields pass through on their way to the caller, in
-// pieces of at most 1 MiB, two per lane, so that one piece is converted or
-// copied out while the next one arrives.  Fields of 4 MiB and more go through
-// four lanes, a host thread each: a single thread is bound by the page faults
-// of the caller's fresh array (a field of 8192 x 1024 took 12 ms through an
-// unpinned copy and a conversion, 2.1 ms this way; 2001 x 203 0.20 and 0.14 ms).
-// Owned by one context (allocated with it, no larger than its fields need) and
-// used by one call at a time.
-class FetchStage {
- public:
-  FetchStage() = default;
-  FetchStage(const FetchStage&) = delete;
-  FetchStage& operator=(const FetchStage&) = delete;
-  ~FetchStage() {
-    for (hipEvent_t ev : done_)
-      if (ev) (void)hipEventDestroy(ev);
-    if (mem_) (void)hipHostFree(mem_);
-  }
-  hipError_t create(size_t fieldBytes) {
-    hipError_t e = hipGetDevice(&device_);
-    if (e != hipSuccess) return e;
-    piece_ = std::min(kPiece, std::max<size_t>((fieldBytes + 255) / 256 * 256, 256));
-    lanes_ = fieldBytes >= kLaneFrom ? kLanes : 1;
-    e = hipHostMalloc(reinterpret_cast<void**>(&mem_), 2 * size_t(lanes_) * piece_, hipHostMallocDefault);
-    for (int i = 0; i < 2 * lanes_ && e == hipSuccess; i++)
-      e = hipEventCreateWithFlags(&done_[i], hipEventDisableTiming);
-    return e;
-  }
-
-  // n values of type T at the device address src to doubles at host, after
-  // the work enqueued on stream.
-  template <class T>
-  hipError_t fetch(hipStream_t stream, const T* src, size_t n, double* host) {
-    const int lanes = n * sizeof(T) >= kLaneFrom ? lanes_ : 1;
-    if (lanes == 1) return lane(0, stream, src, 0, n, host);
-    std::atomic<int> bad{int(hipSuccess)};
-    auto part = [&](int t) {
-      const size_t a = n * size_t(t) / size_t(lanes), b = n * size_t(t + 1) / size_t(lanes);
-      const hipError_t e = lane(t, stream, src, a, b, host);
-      if (e != hipSuccess) bad = int(e);
-    };
-    std::thread team[kLanes];
-    int started = 1;
-    try {
-      for (; started < lanes; started++)
-        team[started] = std::thread([&, t = started] {
-          if (hipSetDevice(device_) == hipSuccess)
-            part(t);
-          else
-            bad = int(hipErrorInvalidDevice);
-        });
-    } catch (const std::system_error&) {  // no more threads: the rest runs here
-    }
-    part(0);
-    for (int t = started; t < lanes; t++) part(t);
-    for (int t = 1; t < started; t++) team[t].join();
-    return hipError_t(bad.load());
-  }
-
- private:
-  static constexpr size_t kPiece = size_t(1) << 20, kLaneFrom = size_t(4) << 20;
-  static constexpr int kLanes = 4;
-  char* mem_ = nullptr;
-  hipEvent_t done_[2 * kLanes] = {};
-  size_t piece_ = 0;
-  int lanes_ = 1, device_ = 0;
-
-  template <class T>
-  hipError_t lane(int t, hipStream_t stream, const T* src, size_t a, size_t b, double* host) {
-    const size_t per = piece_ / sizeof(T);
-    T* buf[2] = {reinterpret_cast<T*>(mem_ + 2 * size_t(t) * piece_),
-                 reinterpret_cast<T*>(mem_ + (2 * size_t(t) + 1) * piece_)};
-    hipEvent_t* ev = done_ + 2 * t;
-    auto start = [&](size_t i, int k) {
-      hipError_t e = hipMemcpyAsync(buf[k], src + i, std::min(per, b - i) * sizeof(T),
-                                    hipMemcpyDeviceToHost, stream);
-      return e == hipSuccess ? hipEventRecord(ev[k], stream) : e;
-    };
-    if (b - a <= per) {
-      hipError_t e = hipMemcpyAsync(buf[0], src + a, (b - a) * sizeof(T), hipMemcpyDeviceToHost, stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(stream);
-      if (e == hipSuccess) std::copy(buf[0], buf[0] + (b - a), host + a);
-      return e;
-    }
-    hipError_t e = start(a, 0);
-    int k = 0;
-    for (size_t i = a; i < b && e == hipSuccess; i += per, k ^= 1) {
-      if (i + per < b) e = start(i + per, k ^ 1);
-      if (e == hipSuccess) e = hipEventSynchronize(ev[k]);
-      if (e == hipSuccess) std::copy(buf[k], buf[k] + std::min(per, b - i), host + i);
-    }
-    // nothing may still be arriving when the stage is used again
-    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
-    return e;
-  }
 };
 
 // Default padding of the population planes (elements).
@@ -247,7 +148,7 @@ class EngineT final : public Engine {
     HIP_TRY(passState_.alloc(4 * sizeof(dev::SolveState)));
     HIP_TRY(redPartial_.alloc(dev::kReducePartials * sizeof(double)));
     HIP_TRY(redOut_.alloc(sizeof(double)));
-    HIP_TRY(stage_.create(9 * D * sizeof(double)));  // the populations are the largest field
+    HIP_TRY(stage_.open(9 * D * sizeof(double)));  // the populations
     return 0;
   }
 

@@ -1,8 +1,9 @@
 """Fields reach the host whole at the sizes where their way changes: below one
-piece of pinned memory (1 MiB), across pieces with a remainder, and from 4 MiB
-on in four parts.  The populations come back as they were uploaded (FP64
-storage: to the last bits of f = w + (f - w)), and a field downloaded twice, or
-reduced on the device, agrees with itself.
+piece of pinned memory (1 MiB), across pieces with a remainder, and, for large
+fields (the last size's in both precisions), in four parts.  The populations
+come back as they were uploaded (FP64 storage: to the last bits of
+f = w + (f - w)), and a field downloaded twice, or reduced on the device,
+agrees with itself.
 """
 import numpy as np
 import pytest
@@ -12,7 +13,8 @@ from komegafoulingmodel_amd import channel, lib
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nX,nY", [(100, 8), (130, 75), (1025, 129), (1500, 467)])
+@pytest.mark.parametrize("nX,nY", [(100, 8), (130, 75), (1025, 129), (1500, 467),
+                                   (2049, 1030)])
 @pytest.mark.parametrize("storage", ["f32", "f64"])
 def test_fields_come_back_whole(nX, nY, storage):
     w = channel.flat_channel(nX, nY, seed=nX)

@@ -527,20 +527,20 @@ int kofm_save_debug(kofm_ctx* ctx, const char* dir);
  * nX is even), steps per pass (1, or 2 for the temporally blocked kernels:
  * k-omega off, nodes_per_lane 1, and block_x is then the tile's node count,
  * 512 (64 x 8), 832 (64 x 13), 640 (128 x 5) or 1856 (64 x 29) with one
- * node per lane and step, or 1024 (64 x 16), 1664 (64 x 26), 1536
- * (128 x 12) or, with 16- or 32-bit storage, 3584 (128 x 28) with two
- * neighbouring nodes per lane; the tile width must divide nX) and the
- * padding (elements,
- * multiple of 64) between the nine population planes in HBM.  The state is preserved and
- * every shape gives bit-identical results.  Until a shape is set, plain steps
- * take two steps per pass where that is the faster for the lattice's size.  No counterpart in the reference,
- * whose work-group is fixed at 128 x 1 (ConstDef.h:70-79). */
+ * node per lane and step, on any width, or 1024 (64 x 16), 1664 (64 x 26),
+ * 1536 (128 x 12) or, with 16- or 32-bit storage, 3584 (128 x 28) with two
+ * neighbouring nodes per lane, where the tile's width divides nX) and the
+ * padding (elements, multiple of 64) between the nine population planes in
+ * HBM.  The state is preserved and every shape gives bit-identical results.
+ * Until a shape is set, plain steps take two steps per pass where that is the
+ * faster for the lattice's size.  No counterpart in the reference, whose
+ * work-group is fixed at 128 x 1 (ConstDef.h:70-79). */
 int kofm_set_launch(kofm_ctx* ctx, int32_t block_x, int32_t nodes_per_lane,
                     int32_t steps_per_pass, int64_t plane_pad);
 
 /* Times the collide-stream kernels over the candidate shapes (about `steps`
  * steps each, on scratch populations at rest) and keeps the fastest; returns
- * the choice and its time per step.  No counterpart in the reference. */
+ * the choice, as kofm_set_launch takes it, and its time per step.  No counterpart in the reference. */
 int kofm_autotune(kofm_ctx* ctx, int32_t steps, int32_t* block_x, int32_t* nodes_per_lane,
                   int32_t* steps_per_pass, int64_t* plane_pad, double* ms_per_step);
 

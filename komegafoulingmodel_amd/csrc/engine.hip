@@ -2060,6 +2060,12 @@ class EngineT final : public Engine {
   static int t2Width(int nodes) {
     return (nodes == 640 || nodes == 1536 || nodes == 3584) ? 128 : 64;
   }
+  // Tiles of one node per lane may be cut by the lattice's edge; node pairs
+  // cover whole tiles only.
+  bool t2Fits(int nodes) const {
+    const bool pairs = nodes == 1024 || nodes == 1536 || nodes == 1664 || nodes == 3584;
+    return t2Tile(nodes) && (!pairs || nX_ % t2Width(nodes) == 0);
+  }
   // (the 128 x 28 tile's LDS planes exceed a work-group's 160 KB with FP64
   // storage)
   static bool t2Tile(int nodes) {
@@ -2202,11 +2208,10 @@ class EngineT final : public Engine {
     if (spp != 1 && spp != 2) return fail(err, "steps per pass must be 1 or 2");
     if (spp == 2 && kSR)
       return fail(err, "the FP32 storage form with FP64 collisions takes one step per pass");
-    if (spp == 2 && (ko_ || npt != 1 || !t2Tile(block) || nX_ % t2Width(block)))
+    if (spp == 2 && (ko_ || npt != 1 || !t2Fits(block)))
       return fail(err, "two steps per pass need k-omega off, nodes_per_lane 1 and a tile "
-                       "(block_x) of 512, 640, 832, 1856, 1024, 1536, 1664 or (16- and 32-bit "
-                       "storage) 3584 nodes whose "
-                       "width divides nX");
+                       "(block_x) of 512, 640, 832 or 1856 nodes, or of 1024, 1536, 1664 or (16- and "
+                       "32-bit storage) 3584 nodes where its width divides nX");
     if (pad < 0 || pad % 64) return fail(err, "plane padding must be a non-negative multiple of 64");
     int rc = relayout(pad, err);
     if (rc) return rc;
@@ -2236,7 +2241,6 @@ class EngineT final : public Engine {
     bestSpp = lbSpp_;
     bestPad = P_ - D_;
     int rc = 0;
-    bool bestOwn = false;
     for (int64_t pad : pads) {
       if (!popsFit(D_ + pad)) continue;
       Buffer a, b;
@@ -2267,15 +2271,11 @@ class EngineT final : public Engine {
             bestNpt = npt;
             bestSpp = 1;
             bestPad = pad;
-            bestOwn = false;
           }
         }
       if (!ko_ && !kSR)
         for (int block : {512, 640, 832, 1856, 1024, 1536, 1664, 3584}) {
-          // of widths that are no multiple of a tile's, the size's own tile (the
-          // launch without a set shape) is a candidate
-          const bool own = nX_ % 64 && block == autoTile();
-          if (!own && (!t2Tile(block) || nX_ % t2Width(block))) continue;
+          if (!t2Fits(block)) continue;
           auto pA = p, pB = p;
           pA.applyIbb = 1;
           launchT2(block, pA, pB, a.as<S>(), b.as<S>());  // warm-up
@@ -2294,7 +2294,6 @@ class EngineT final : public Engine {
             bestNpt = 1;
             bestSpp = 2;
             bestPad = pad;
-            bestOwn = own;
           }
         }
     }
@@ -2302,14 +2301,7 @@ class EngineT final : public Engine {
     (void)hipEventDestroy(e1);
     HIP_TRY(hipGetLastError());
     if (rc) return rc;
-    if (!bestOwn) return setLaunch(bestBlock, bestNpt, bestSpp, bestPad, err);
-    // the launch without a set shape, reported as the one-step shape that
-    // kofm_set_launch takes on such a width
-    bestBlock = 256;
-    bestSpp = 1;
-    rc = setLaunch(bestBlock, 1, 1, bestPad, err);
-    if (!rc) autoLaunch_ = true;
-    return rc;
+    return setLaunch(bestBlock, bestNpt, bestSpp, bestPad, err);
   }
 
  private:

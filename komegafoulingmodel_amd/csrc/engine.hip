@@ -2048,7 +2048,7 @@ class EngineT final : public Engine {
     auto p = lbParams(0);
     p.applyIbb = apply;
     p.saveMacros = 0;
-    launchLBBlock<false>(autoLaunch_ ? 256 : lbBlock_, lbNpt_, p, src, dst);
+    launchLBBlock<false>(oneStepWidth(), lbNpt_, p, src, dst);
   }
 
   // The temporally blocked kernels, selected by the tile's node count: one
@@ -2135,6 +2135,18 @@ class EngineT final : public Engine {
     if (n < 600000) return 832;
     return sizeof(S) == 4 && nX_ % 128 == 0 && n >= 4000000 ? 1536 : 1856;
   }
+  // The work-group width of one plain step per pass (single steps, FP32 storage
+  // with FP64 collisions, large 16-bit lattices of odd width).  Measured with no
+  // shape set, 256 against 512 lanes, us a step: FP32 2001 x 203 7.6 and 10.8,
+  // 1024 x 128 5.4 and 5.9, 2048 x 512 14.8 and 15.9, 3001 x 700 26.2 and 26.7;
+  // from about 3 million nodes on the wider one is ahead (4096 x 1024 60.7 and
+  // 59.6, FP64 120 and 116; 8192 x 1024 122 and 117, FP64 239 and 228, FP32 with
+  // saved macros 141 and 137), and with FP64 storage on rows that 512 divides
+  // (1024 x 128 7.3 and 6.7, 1024 x 256 9.8 and 9.4; 2001 x 203 12.3 and 13.6).
+  int oneStepWidth() const {
+    if (!autoLaunch_) return lbBlock_;
+    return int64_t(nX_) * nY_ >= 3000000 || (sizeof(S) == 8 && nX_ % 512 == 0) ? 512 : 256;
+  }
   int stepsPerPass() const { return autoLaunch_ ? (autoTile() ? 2 : 1) : lbSpp_; }
 
   // Two plain steps in one pass (k-omega off); the macros, if asked for,
@@ -2156,7 +2168,7 @@ class EngineT final : public Engine {
     if (ko_)
       launchLBBlock<true>(lbBlock_, lbNpt_, p, cur(), other());
     else
-      launchLBBlock<false>(autoLaunch_ ? 256 : lbBlock_, lbNpt_, p, cur(), other());
+      launchLBBlock<false>(oneStepWidth(), lbNpt_, p, cur(), other());
     curBuf_ ^= 1;
     preIbb_ = true;
     stepCount_++;

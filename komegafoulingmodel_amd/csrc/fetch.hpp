@@ -131,10 +131,15 @@ class PinnedLanes {
 
 // The way of a context's fields: through a lane piece by piece, so that one
 // piece is converted or copied out while the next one arrives.  Fields of
-// 4 MiB and more go through four lanes, a host thread each: a single thread is
-// bound by the page faults of the caller's fresh array (a field of 8192 x 1024
-// took 12 ms through an unpinned copy and a conversion, 2.1 ms this way; 2001 x
-// 203 0.20 and 0.14 ms).  Without a lane a field is copied unpinned.
+// 8 MiB (on the device) and more go through four lanes, a host thread each: a
+// single thread is bound by the page faults of the caller's fresh arrays.  The
+// line lies where that first pays.  One lane against four, us a field, into an
+// array whose pages are there and, in brackets, three fields into new pages:
+// FP32 4 MiB 176 and 236, 8 MiB 318 and 400 (2480 and 2080), 12 MiB 466 and 508
+// (5280 and 2990); FP64 6 MiB 268 and 308 (2130 and 1420), 8 MiB 328 and 341,
+// 16 MiB 646 and 602.  A field of 8192 x 1024 took 12 ms through an unpinned copy
+// and a conversion, 2.2 ms this way; 2001 x 203 0.20 and 0.14 ms.  Without a lane
+// a field is copied unpinned.
 class FetchStage {
  public:
   // The stage of a context on the current device whose largest field has so
@@ -181,7 +186,7 @@ class FetchStage {
 
  private:
   using Lane = PinnedLanes::Lane;
-  static constexpr size_t kLaneFrom = size_t(4) << 20;
+  static constexpr size_t kLaneFrom = size_t(8) << 20;
   static constexpr int kLanes = 4;
   std::shared_ptr<PinnedLanes> pinned_;
   int device_ = 0;

@@ -640,12 +640,14 @@ int kofm_ensemble_set_block(kofm_ensemble* e, int32_t block_x);
  * or, with 16- or 32-bit storage, 3584 (128 x 28); every member's nX a
  * multiple of the tile width.  Results are bit-identical for every shape. */
 int kofm_ensemble_set_launch(kofm_ensemble* e, int32_t block_x, int32_t steps_per_launch);
-/* Members are packed (largest first) into groups whose population arrays
- * (both buffers) total at most `bytes`; kofm_ensemble_step advances each
- * group through all its steps before the next, so a group that fits the
- * last-level cache (256 MB on MI355X) runs from it.  0 puts every member in
- * one launch per step.  The default is 160 MiB.  *groups (may be NULL)
- * receives the number of groups.  Results do not depend on the grouping. */
+/* Members are packed (largest first) into groups whose working sets total at
+ * most `bytes` (a member's population arrays, both buffers, and with k-omega
+ * its FP64 fields and solver vectors, 42 values per node);
+ * kofm_ensemble_step advances each group through all its steps before the
+ * next, so a group that fits the last-level cache (256 MB on MI355X) runs from
+ * it.  0 puts every member in one launch per step.  The default is 160 MiB, and
+ * 0 for members with k-omega.  *groups (may be NULL) receives the number of
+ * groups.  Results do not depend on the grouping. */
 int kofm_ensemble_set_cache_budget(kofm_ensemble* e, int64_t bytes, int32_t* groups);
 /* Times `steps` ensemble steps for each launch shape (one step per launch
  * with 256 or 512 wide groups; with k-omega off also the two-step 832 and

@@ -707,8 +707,10 @@ class EngineT final : public Engine {
 
   int download(int field, double* host, std::string& err) override {
     if (field == KOFM_FIELD_F) {
-      // populations in the reference layout; the buffer of a small lattice is
-      // kept for the next call (an allocation costs more than its copy)
+      // populations in the reference layout; a buffer of up to 64 MiB is kept
+      // for the next call (allocated each time, us a call: 256 x 64 157 instead
+      // of 115, 1024 x 200 951 and 794, 2048 x 400 2370 and 2080; larger ones would
+      // gain as much as the copy takes but hold 72 bytes a node)
       const size_t n = 9 * size_t(D_), bytes = n * sizeof(double);
       Buffer tmp;
       Buffer& out = bytes <= kKeepExport ? export_ : tmp;
@@ -1232,12 +1234,16 @@ class EngineT final : public Engine {
   // fields, the per-step done flags and iteration counts (device, pinned
   // host copy), and the steps still to run one at a time after a rollback
   static constexpr int kKoBatch = 8, kKoBatchMaxIters = 16;
-  // Iterations each step of a batch is given: the most that a step of the
-  // last 128 needed; while that is above 4 (a start-up transient) the last
-  // solve's and two more, with the most of the last 16 kept.  A pass that finds
-  // its system done still costs its launch, 4.5 us in a chain (13.5 per spare
-  // iteration, of a 110 us step on 2000 x 204); one step in 128 that needs more
-  // costs a rollback of eight.
+  // Iterations each step of a batch is given: the most that a step of this and
+  // the last window of 128 needed; while that is above 4 (a start-up transient)
+  // the last solve's and two more, in windows of 16.  A pass that finds its
+  // system done still costs its launch, 4.5 us in a chain (13.5 per spare
+  // iteration, of a 110 us step on 2000 x 204); a step that needs more costs a
+  // rollback of eight, on flat walls once in thousands of steps, on curved ones
+  // at most once in 64.  Two spare iterations always took 102 us a step instead of
+  // 83 on the flat 2000 x 204, 96 and 80 on a wavy 1024 x 128, 173 and 180 on a
+  // wavy 2000 x 204 (31 rollbacks in 2048 steps); windows of 32 or 512, of 4 or 64
+  // in a transient, and a transient from 2 or 16 on lie within 7 % of these.
   int predIters_ = 1, predWindow_ = 1, predAge_ = 0;
   void noteIterations(int iters, int steps) {
     predWindow_ = std::max(predWindow_, iters);
@@ -2124,9 +2130,11 @@ class EngineT final : public Engine {
   // 600 26.3 -> 18.5 (47.9 -> 30.1) with 64 x 29, 8192 x 1024 FP32 119 -> 76 with
   // the node pairs of 128 x 12 (94 with 64 x 29).  FP16: 1984 x 203 7.9 -> 4.7 and
   // 1472 x 467 11.1 -> 7.9 with 64 x 13, 2048 x 600 13.2 -> 10.0 with the node pairs
-  // of 64 x 26 (12.0 with 64 x 13); a large odd width is no faster in two-step
-  // tiles (4096 x 512: 17.7, 18.6 to 21.8).  A small lattice needs many blocks, a
-  // large one little ring.
+  // of 64 x 26 (12.0 with 64 x 13); above a million nodes the tiles of one node per
+  // lane, the only ones that a width no multiple of 64 can take, are no faster
+  // than one step per pass (4096 x 512: 17.7, 18.6 to 21.8).  A small lattice needs
+  // many blocks, a large one little ring.  How far a row's last tile is cut does
+  // not enter: 257 x 61, whose last tile holds one column, gains like the others.
   int autoTile() const {
     if (ko_ || kSR) return 0;
     const int64_t n = int64_t(nX_) * nY_;
@@ -3242,7 +3250,7 @@ class EnsembleT final : public Ensemble {
   int block_ = 512;
   int spp_ = 1;
   bool ko_ = false;  // every member runs k-omega
-  // working-set bytes per group; 0 puts every member in one launch.  The
+  // bytes per group (regroup); 0 puts every member in one launch.  The
   // default fits the 256 MB last-level cache with room to spare; k-omega
   // members, whose step is a dozen launches for a group of any size, start as
   // one group (six channels of 1.3 million nodes: 427 us a step, 678 in

@@ -24,7 +24,7 @@
 // are the first residual itself, so r is never overwritten in its first buffer
 // (later residuals alternate between two others) and the first iteration,
 // which is the only one for most steady steps, moves 6 + 7 + 6 planes instead
-// of 10 + 8 + 7; s is recomputed in XR.
+// of 10 + 7 + 8; s is recomputed in XR.
 #pragma once
 #include "kernels.hpp"
 
@@ -119,10 +119,12 @@ __device__ __forceinline__ bool chunkOf(const Strips& s, int nX, int nY, Chunk& 
   return true;
 }
 
-// A sum carried with its rounding error (Knuth's two-sum): the passes' dot
-// products then do not depend on how the lattice is cut into blocks, which
+// A sum carried with its rounding error (Knuth's two-sum): how the lattice is
+// cut into blocks then changes the passes' dot products by little more than
+// their last rounding (the errors themselves are added up plainly), which
 // ill-conditioned rows (fouled walls) would otherwise feel from the third
-// iteration on.  The passes wait for memory; the extra additions are free.
+// iteration on.  The passes wait for memory; plain sums measured 0.6 to 1 us
+// less of a pass's 5 to 40.
 struct Sum {
   double hi, lo;
   __device__ __forceinline__ void add(double x) {

@@ -534,8 +534,8 @@ class Lattice:
 
 
 class Ensemble:
-    """Several Lattice objects (same storage, k-omega off) stepped together,
-    one launch per step."""
+    """Several Lattice objects (same storage, k-omega all off or all on) stepped
+    together, their launches shared."""
 
     def __init__(self, members):
         self.lib = load()
@@ -575,8 +575,9 @@ class Ensemble:
         return b.value, s.value, g.value, ms.value
 
     def set_cache_budget(self, nbytes: int) -> int:
-        """Groups the members under a population-byte budget (0: one group);
-        returns the number of groups."""
+        """Groups the members under a budget of working-set bytes (0: one group,
+        the default with k-omega; 160 MiB without); returns the number of
+        groups."""
         g = C.c_int32()
         self._check(self.lib.kofm_ensemble_set_cache_budget(self.h, nbytes, C.byref(g)))
         return g.value

@@ -1330,10 +1330,15 @@ class EngineT final : public Engine {
   // captured objective-run and adjoint segments (their launches bake in the
   // checkpoint-segment and adjoint buffers, the objective nodes and the
   // parameters)
-  std::vector<std::pair<std::vector<int64_t>, hipGraphExec_t>> sweepGraphs_;
+  struct SweepGraph {
+    std::vector<int64_t> key;
+    hipGraphExec_t exec;
+    int swaps;  // 1: its passes leave the populations in the other buffer
+  };
+  std::vector<SweepGraph> sweepGraphs_;
 
   void dropSweeps() {
-    for (auto& g : sweepGraphs_) (void)hipGraphExecDestroy(g.second);
+    for (auto& g : sweepGraphs_) (void)hipGraphExecDestroy(g.exec);
     sweepGraphs_.clear();
   }
 
@@ -1725,17 +1730,20 @@ class EngineT final : public Engine {
   }
 
   // Launches the graph captured for key, capturing it from enqueue() the
-  // first time.  A capture leaves curBuf_/preIbb_ where the enqueued steps
-  // put them; a replay advances them by `steps` plain steps.
+  // first time.  A capture leaves curBuf_/preIbb_ where the enqueued passes
+  // put them, and so does a replay: the buffers are swapped by each pass, which
+  // may hold two of the `steps`.
   template <class F>
   int replay(const std::vector<int64_t>& key, F&& enqueue, int steps, std::string& err) {
     hipGraphExec_t exec = nullptr;
     for (auto& g : sweepGraphs_)
-      if (g.first == key) exec = g.second;
-    if (exec) {
-      curBuf_ ^= steps & 1;
-      if (steps > 0) preIbb_ = true;
-    } else {
+      if (g.key == key) {
+        exec = g.exec;
+        curBuf_ ^= g.swaps;
+        if (steps > 0) preIbb_ = true;
+      }
+    if (!exec) {
+      const int buf0 = curBuf_;
       hipGraph_t graph = nullptr;
       HIP_TRY(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
       enqueue();
@@ -1743,7 +1751,7 @@ class EngineT final : public Engine {
       hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
       (void)hipGraphDestroy(graph);
       HIP_TRY(e);
-      sweepGraphs_.push_back({key, exec});
+      sweepGraphs_.push_back({key, exec, buf0 ^ curBuf_});
     }
     HIP_TRY(hipGraphLaunch(exec, stream_));
     return 0;

@@ -258,22 +258,35 @@ def test_torch_autograd_returns_the_adjoint():
     P2.close()
 
 
-def test_adjoint_is_independent_of_the_launch_shape():
-    """With the two-step launch shape the objective run steps in pairs before
-    the window and the recompute runs the two-step kernel that also writes
-    the middle state; J and the gradient are bit-identical to one-step
-    launches."""
+@pytest.mark.parametrize("nX,storage,interval", [
+    (192, "f32", 16), (192, "f32", 18), (192, "f16", 3), (255, "f64", 13), (255, "f32", 6)])
+def test_adjoint_is_independent_of_the_launch_shape(nX, storage, interval):
+    """Where plain steps go in pairs (by a set shape, or without one) the
+    objective run steps in pairs before the window and the recompute runs the
+    two-step kernel that also writes the middle state, on whole tiles and on
+    rows whose last tile has 63 columns, in intervals of an odd and an even
+    number of pairs with and without a single step at their end.  J, the
+    gradients by the wall points and by the links' q, and the state the run
+    leaves behind are bit-identical to one-step launches, also when the run is
+    repeated from the same state, with every interval's graph captured."""
     res = []
-    for shape in (None, (832, 1, 64, 2)):
-        P = _problem("f32")
-        th = P.initial_theta()
+    for shape in ((256, 1, 1088, 1), None, (832, 1, 64, 2)):
+        P = _problem(storage, nX=nX, period=nX / 2.0, interval=interval)
+        L = P.lattice()
         if shape:
-            P.lattice().set_launch(*shape)
-        J = P.objective(th)
-        res.append((J, P.gradient()))
+            L.set_launch(*shape)
+        P.build(P.initial_theta())
+        f0 = L.download("f")
+        for _ in range(2):
+            L.upload_state(f0)
+            J = L.objective_run(P.steps, P.interval, P.window, shear_weight=P.shear_weight)
+            f = L.download("f")
+            res.append((np.array([J]), f) + tuple(L.adjoint()))
         P.close()
-    assert res[0][0] == res[1][0]
-    assert np.array_equal(res[0][1], res[1][1])
+    assert np.max(np.abs(res[0][2])) > 0
+    for r in res[1:]:
+        for got, ref in zip(r, res[0]):
+            assert np.array_equal(got, ref)
 
 
 def test_frozen_turbulence_adjoint_reduces_to_the_laminar_adjoint():

@@ -234,6 +234,9 @@ class EngineT final : public Engine {
       markUnitSpacing(mask_, dX_);
       HIP_TRY(hipGetLastError());
     }
+    gaps_ = findGaps();
+    emptySolids();
+    HIP_TRY(hipGetLastError());
     haveGeo_ = true;
     return 0;
   }
@@ -432,6 +435,7 @@ class EngineT final : public Engine {
     int rc = refreshWallDerived(C, geo_, err);
     if (!rc) rc = uploadShear(err);
     if (rc) return rc;
+    gaps_ = findGaps();
     gen_++;
     dropGraphs();
     run_.valid = false;
@@ -440,6 +444,7 @@ class EngineT final : public Engine {
       auto p = lbParams(0);
       hipLaunchKernelGGL((dev::lbImportF<S, R>), gridXY(XF_), dim3(dev::kBlockX), 0, stream_,
                          (const double*)keep.as<double>(), fA_.as<S>(), p);
+      emptySolids();
       HIP_TRY(hipGetLastError());
       preIbb_ = false;
     }
@@ -1169,6 +1174,7 @@ class EngineT final : public Engine {
     int rc = reserve(seg_, K + 1, state, err);
     if (!rc) rc = adjointBuffers(err);
     if (rc) return rc;
+    emptySegments();
     dev::AdjointBuffers abuf{ibbNodes_.as<int32_t>(), upBar_.as<void>(), qBar_.as<double>(),
                              nIbbNodes_};
     dev::ObjectiveNodes on = objNodes();
@@ -1210,6 +1216,7 @@ class EngineT final : public Engine {
   Buffer K_, O_, nut_, S_, wallD_, Dk_, Do_, F1_, dkdo_, dX_, Ak_, Ao_;
   Buffer ntype_, dX0_;  // node types and clean-wall spacings (moving-wall update)
   std::vector<double> wallC0_;  // the wall points of the built (clean) geometry
+  bool gaps_ = false;           // links read solid nodes' slots (lbSolidSlots)
   bool wallsMoved_ = false;     // the walls were updated since the geometry was built
   Buffer Kprev_, Oprev_;  // k, omega at the start of the step (restart point)
   Buffer kr_[2][3], kp_[2][2], kv_[2][2], kt_[2];  // FP64 BiCGStab vectors, [0] = k
@@ -1502,6 +1509,7 @@ class EngineT final : public Engine {
     if (!rc) rc = reserve(tape_, K + 1, tapeBytes(), err);
     if (!rc) rc = adjointBuffers(err);
     if (rc) return rc;
+    emptySegments();
     if (kaBuf_.bytes() < kAPlanes * d8) HIP_TRY(kaBuf_.alloc(kAPlanes * d8));
     if (koSave_.bytes() < 6 * d8 + 3 * dr) HIP_TRY(koSave_.alloc(6 * d8 + 3 * dr));
     char* sv = koSave_.as<char>();
@@ -1966,6 +1974,7 @@ class EngineT final : public Engine {
     p.saveMacros = (options & KOFM_OPTION_SAVE_MACRO_FIELDS) || ko_ ? 1 : 0;
     p.applyIbb = preIbb_ ? 1 : 0;
     p.seed = stepCount_;
+    p.gaps = gaps_ ? 1 : 0;
     return p;
   }
 
@@ -2018,9 +2027,38 @@ class EngineT final : public Engine {
     auto p = lbParams(0);
     hipLaunchKernelGGL((dev::lbImportF<S, R>), gridXY(XF_), dim3(dev::kBlockX), 0, stream_,
                        (const double*)tmp.as<double>(), fA_.as<S>(), p);
+    emptySolids();
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(stream_));
     return 0;
+  }
+
+  // Whether a link with q > 1/2 reads a solid node's slot (its node lies in a
+  // gap one node wide along the link).
+  bool findGaps() const {
+    for (size_t l = 0; l < geo_.ibb.size(); l++) {
+      if (!(geo_.ibbQ[l] > 0.5)) continue;
+      const int d = int(geo_.ibb[l] / D_);
+      const int64_t node = geo_.ibb[l] - int64_t(d) * D_;
+      const int x = int(node % XF_) - Lattice::cx[d];
+      const int64_t up = (x + nX_) % nX_ + (node / XF_ - Lattice::cy[d]) * XF_;
+      if (up >= 0 && up < D_ && (geo_.nType[size_t(up)] & kMSolid)) return true;
+    }
+    return false;
+  }
+  // After the populations or the node types have changed.
+  void emptySolids() {
+    if (gaps_)
+      hipLaunchKernelGGL((dev::lbSolidSlots<S, R>), gridXY(nX_), dim3(dev::kBlockX), 0, stream_,
+                         fA_.as<S>(), fB_.as<S>(), (const uint16_t*)mask_.as<uint16_t>(), lbParams(0));
+  }
+  // The same for the adjoint's recomputed states.
+  void emptySegments() {
+    if (gaps_)
+      for (auto& b : seg_)
+        hipLaunchKernelGGL((dev::lbSolidSlots<S, R>), gridXY(nX_), dim3(dev::kBlockX), 0, stream_,
+                           b->template as<S>(), (S*)nullptr, (const uint16_t*)mask_.as<uint16_t>(),
+                           lbParams(0));
   }
 
   template <bool KO, int BX, int NPT>
@@ -2220,6 +2258,7 @@ class EngineT final : public Engine {
       auto p = lbParams(0);
       hipLaunchKernelGGL((dev::lbImportF<S, R>), gridXY(XF_), dim3(dev::kBlockX), 0, stream_,
                          (const double*)tmp.as<double>(), fA_.as<S>(), p);
+      emptySolids();
       HIP_TRY(hipGetLastError());
       HIP_TRY(hipStreamSynchronize(stream_));
       preIbb_ = false;

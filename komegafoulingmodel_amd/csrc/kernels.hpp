@@ -174,6 +174,7 @@ struct LBParams {
   int saveMacros;
   int applyIbb;
   uint32_t seed;  // the step's index: the stochastic rounding of FP32 stores with FP64 collisions
+  int gaps;       // wall links read solid nodes' slots (lbSolidSlots)
 };
 
 // 1-D equilibrium deviation: phi(c,u) - w1(c)
@@ -202,7 +203,8 @@ __device__ __forceinline__ R geq(int i, R drho, R rho, R ux, R uy) {
 // value and the node's own incoming value, q > 1/2 between the bounced
 // value and the reversed value streamed to the upstream neighbour).
 // up(d) returns the stored slot rev(d) of the node one step upstream
-// (x - c_d), read only for q > 1/2.
+// (x - c_d), read only for q > 1/2; in a gap one node wide along d that is a
+// solid node's slot (lbSolidSlots).
 template <class R, class Up>
 __device__ __forceinline__ void ibbCorrectWith(R (&g)[9], const R* __restrict__ q8, Up&& up) {
   R nv[9];
@@ -438,6 +440,12 @@ __device__ __forceinline__ S toStored(R g, int slot) {
   if constexpr (Scaled<S>::value) g *= R(scale16(slot));
   return static_cast<S>(g);
 }
+// What the slots of a solid node hold: f = 0, the reference's never-written
+// entries.
+template <class S, class R>
+__device__ __forceinline__ S emptySlot(int slot) {
+  return toStored<S, R>(R(-wgt(slot)), slot);
+}
 template <class S, class R>
 __device__ __forceinline__ R fromStored(S v, int slot) {
   R g = static_cast<R>(v);
@@ -621,7 +629,13 @@ __device__ __forceinline__ void t2Tile(const S* __restrict__ src, S* __restrict_
     x = x < 0 ? x + pA.nX : (x >= pA.nX ? x - pA.nX : x);
     const size_t gi = size_t(x) + size_t(pA.XF) * y;
     const uint32_t m = mask[gi];
-    if (m & kSolid) continue;
+    if (m & kSolid) {
+      if (pA.gaps) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) mid[i][r] = emptySlot<S, R>(i);
+      }
+      continue;
+    }
     R g[9];
     loadNode<S, R>(g, src, gi, x, y, m, ibbIdx, ibbQ, pA);
     collideNode<R, false, kWideMoments<S, R>>(g, gi, rhoOut, uxOut, uyOut, none, pA);
@@ -789,8 +803,16 @@ __device__ __forceinline__ void t2pStep1(const T2PIn<S>& in, int q,
   const KOFields none{nullptr, nullptr, nullptr, nullptr, nullptr};
   if (in.y < 0) return;
   const uint32_t m[2] = {in.mm & 0xFFFFu, in.mm >> 16};
-  if ((m[0] & kSolid) && (m[1] & kSolid)) return;
   const int rx0 = 2 * (q % (Sh::RX / 2)), ry = q / (Sh::RX / 2);
+  if (pA.gaps) {
+#pragma unroll
+    for (int n = 0; n < 2; n++)
+      if (m[n] & kSolid) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) mid[i][(rx0 + 2) + LX * (ry + 1) + n] = emptySlot<S, R>(i);
+      }
+  }
+  if ((m[0] & kSolid) && (m[1] & kSolid)) return;
   const size_t g0 = size_t(in.xa) + size_t(pA.XF) * in.y;
   R g[2][9];
 #pragma unroll
@@ -1084,6 +1106,26 @@ __global__ __launch_bounds__(kBlockX) void lbImportF(const double* __restrict__ 
 #pragma unroll
   for (int i = 0; i < 9; i++)
     storeDev<S, R>(dst, gi + size_t(p.P) * i, i, R(in[gi + size_t(p.D) * i] - wgt(i)), 0, p.P);
+}
+
+// Empties the slots of every solid node of a (and b, if given).  No step writes
+// them, but a link with q > 1/2 whose node has walls on both sides reads one:
+// where there are such links (LBParams::gaps) both population buffers are kept
+// this way, and the two-step kernels fill the solid cells of their LDS tiles.
+template <class S, class R>
+__global__ __launch_bounds__(kBlockX) void lbSolidSlots(S* __restrict__ a, S* __restrict__ b,
+                                                        const uint16_t* __restrict__ mask,
+                                                        LBParams<R> p) {
+  const int x = blockIdx.x * kBlockX + threadIdx.x;
+  const int y = blockIdx.y;
+  if (x >= p.nX) return;
+  const size_t gi = size_t(x) + size_t(p.XF) * y;
+  if (!(mask[gi] & kSolid)) return;
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    a[gi + size_t(p.P) * i] = emptySlot<S, R>(i);
+    if (b) b[gi + size_t(p.P) * i] = emptySlot<S, R>(i);
+  }
 }
 
 // Macros from populations (Calc_Ro_J lbKernels.cl:137-164, used on upload).

@@ -32,7 +32,8 @@ def _run(w, storage, one_step):
     (65, 40, "f32"), (127, 33, "f64"), (129, 50, "f16"),     # below 50,000 nodes
     (1281, 45, "f32"), (1343, 52, "bf16"), (705, 90, "f64"),  # below 600,000
     (1985, 310, "f32"), (1857, 330, "f64"),                   # above
-    (2049, 490, "f16"), (2112, 480, "f16")])                  # 16-bit, above a million
+    (2049, 490, "f16"), (2112, 480, "f16"), (2112, 480, "bf16"),  # 16-bit, above a million
+    (4096, 980, "f32")])                                      # node pairs of 128 x 12
 def test_default_launch_matches_one_step_per_pass(nX, nY, storage):
     w = channel.fouled_channel(nX, nY, Fval=1e-5, seed=nX, amp=(0.0, 8.0 * nY / 1024.0))
     a, b = _run(w, storage, False), _run(w, storage, True)

@@ -198,10 +198,11 @@ def test_komega_graph_steps_match_eager_launches():
 
 def test_komega_batches_and_their_rollback_match_eager_launches():
     """Batches of 8 k-omega steps replayed from one graph with one poll of
-    the solver state: each step is provisioned the last solve's iterations
-    plus 2.  From the initial state the first solves need more than that, so
-    the first batch rolls back to its checkpoint and runs one step at a time;
-    later batches run whole.  Both end bit-identical to eager launches."""
+    the solver state: each step is given the most iterations that a recent
+    step needed (one before any solve).  From the initial state the first
+    solves need more than that, so the first batch rolls back to its
+    checkpoint and runs one step at a time; later batches run whole.  Both end
+    bit-identical to eager launches."""
     w = _mini_wavy_ko()
     La, _ = make_pair(w, "f32")
     Lb, _ = make_pair(w, "f32")
